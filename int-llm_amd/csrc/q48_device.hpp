@@ -61,6 +61,31 @@ __device__ __forceinline__ int64_t q48_mul_shr(int64_t a, int64_t b)
     return (int64_t)((hi << (64 - S)) | (uint64_t)(mid >> (S - 32)));
 }
 
+// FP64 arithmetic of the calling wave rounds toward minus infinity from here
+// to the end of the kernel (MODE bits 3:2; FP32 keeps its own rounding).  In
+// that mode one fused multiply-add is an exact truncated fixed-point product:
+// for integers a, b and M = 2^52 or 1.5 2^52, fma(a, b 2^-s, M) = M +
+// floor(a b / 2^s) as long as the sum stays in [2^52, 2^53), where doubles
+// are the integers, and a running sum there takes one per term.  Rounding to
+// nearest needs five dependent operations for the same value (product,
+// floor, remainder, floor, add).  Called at the top of every kernel that
+// uses q48_inv_sqrt, q48_exp_small (q48_safe_exp, q48_sigmoid, q48_silu),
+// q48_recip or q48_divisor_of / q48_div_by, which are written for this mode;
+// the general divisions (q48_div, q48_divs_128_64) are exact in either: their
+// estimates are corrected by integer remainders.  The clobber keeps loads,
+// and so the arithmetic on what they load, below the switch.
+__device__ __forceinline__ void q48_round_down()
+{
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 2" ::: "memory");
+}
+
+// The integer v of a double v + 2^52 (0 <= v < 2^52), from its word; as a
+// word, -1 for 2^52 - 1/2.
+__device__ __forceinline__ uint64_t q48_word_m52(double h)
+{
+    return (uint64_t)__builtin_bit_cast(int64_t, h) - 0x4330000000000000ull;
+}
+
 // Constants computed by fp_math_init (fp_math.h:833-858) on the device at
 // context creation: FP_PI, fp_cordic_gain, fp_cordic_angles[48].
 struct q48_consts {
@@ -308,22 +333,16 @@ __device__ __forceinline__ int64_t q48_div(int64_t a, int64_t b)
     return (int64_t)q48_divs_128_64(num, b);
 }
 
-// The nearest integer to 0 <= v < 2^51, minus 1, from the FP64 word of v + 2^52
-// (whose low 52 bits are that integer); as a word, -1 for v below 1/2.
-__device__ __forceinline__ uint64_t q48_round_m1(double v)
-{
-    return (uint64_t)__builtin_bit_cast(int64_t, v + 0x1p52) - 0x4330000000000001ull;
-}
-
 // floor(2^96 / r) = fp_div(ONE, r) for 2^48 <= r < 2^63: the reciprocal in
 // fp_exp of a negative argument and in fp_sigmoid (fp_math.h:516-523 with a
-// = ONE).  y = 1 / r from the hardware reciprocal and two Newton steps has a
-// relative error of a few units of 2^-53 (from any first approximation
-// within 2^-20), so qe = y 2^96 is within 1/16 of 2^96 / r <= 2^48 and q0 =
-// round(qe) - 1 is the quotient or one less.  The remainder 2^96 - q0 r then
-// lies in [0, 2 r), below 2^64, so its low word 0 - q0 r (mod 2^64) is the
-// remainder itself and one compare finishes the quotient.  A remainder that
-// does not settle (an FP64 unit outside those bounds) goes to q48_div.
+// = ONE).  FP64 rounds down (q48_round_down).  y = 1 / r from the hardware
+// reciprocal and two Newton steps has a relative error of a few units of
+// 2^-52 (from any first approximation within 2^-20), so qe = y 2^96 is within
+// 1/4 of 2^96 / r <= 2^48 and q0 = floor(qe - 1/2), the fused y 2^96 + (2^52 -
+// 1/2) rounded down, is the quotient or one less.  The remainder 2^96 - q0 r
+// then lies in [0, 2 r), below 2^64, so its low word 0 - q0 r (mod 2^64) is
+// the remainder itself and one compare finishes the quotient.  A remainder
+// that does not settle (an FP64 unit outside those bounds) goes to q48_div.
 __device__ __forceinline__ int64_t q48_recip(int64_t r)
 {
     const uint64_t u = (uint64_t)r;
@@ -331,7 +350,7 @@ __device__ __forceinline__ int64_t q48_recip(int64_t r)
     double y = __builtin_amdgcn_rcp(rd);
     y = __builtin_fma(y, __builtin_fma(-rd, y, 1.0), y);
     y = __builtin_fma(y, __builtin_fma(-rd, y, 1.0), y);
-    const uint64_t q0 = q48_round_m1(y * 0x1p96);
+    const uint64_t q0 = q48_word_m52(__builtin_fma(y, 0x1p96, 0x1p52 - 0.5));
     const uint64_t rem = (uint64_t)0 - q0 * u;
     const bool up = rem >= u;
     if (rem - (up ? u : 0) >= u)
@@ -362,9 +381,10 @@ __device__ __forceinline__ q48_divisor q48_divisor_of(int64_t d)
 }
 
 // fp_div(e, d) (fp_math.h:508-524) for a divisor from q48_divisor_of.  For 0 <=
-// e <= lim the quotient e 2^48 / d is at most 2^48, e is exact in FP64, qe =
-// e y48 is within 0.1 of the quotient, q0 = round(qe) - 1 is it or one less,
-// and the remainder e 2^48 - q0 d, in [0, 2 d), is its own low word, as in
+// e <= lim the quotient e 2^48 / d is at most 2^48, e is exact in FP64, e y48
+// is within 1/4 of the quotient, q0 = floor(e y48 - 1/2), one fused operation
+// rounded down, is it or one less (-1 for a quotient estimate below 1/2), and
+// the remainder e 2^48 - q0 d, in [0, 2 d), is its own low word, as in
 // q48_recip.  (With lim = 0, e = 0 gives q0 = -1, remainder d and quotient 0,
 // which is fp_div(0, d) for every d != 0.)  Any other e goes to q48_div.
 __device__ __forceinline__ int64_t q48_div_by(int64_t e, const q48_divisor &v)
@@ -372,7 +392,7 @@ __device__ __forceinline__ int64_t q48_div_by(int64_t e, const q48_divisor &v)
     if ((uint64_t)e > v.lim)
         return q48_div(e, (int64_t)v.d);
     const double ed = __builtin_bit_cast(double, (uint64_t)e | 0x4330000000000000ull) - 0x1p52;
-    const uint64_t q0 = q48_round_m1(ed * v.y48);
+    const uint64_t q0 = q48_word_m52(__builtin_fma(ed, v.y48, 0x1p52 - 0.5));
     const uint64_t rem = ((uint64_t)e << 48) - q0 * v.d;
     const bool up = rem >= v.d;
     if (rem - (up ? v.d : 0) >= v.d)
@@ -453,37 +473,39 @@ __device__ __forceinline__ int64_t q48_inv_sqrt(int64_t x)
         y = y1;
         i = 1;
     }
-    // Steps 1..7 on exact doubles, straight-line.  y, y2 = floor(y^2 /
-    // 2^48), xy2 = floor(xn y2 / 2^48), the factor and the next y are
-    // integers below 2^53 while y < 2^49 (xn < 2^50), and each truncated
-    // product a b / 2^s (|a b| <= 2^(s + 52)) is exact:
-    //   with bs = b 2^-s (exact), P = a bs = RN(a b) 2^-s has ulp(P) <= 1,
-    //   so a b 2^-s lies in [f - 1, f + 1) for f = floor(P), and
-    //   fma(a, bs, -f) = (a b - f 2^s) 2^-s exactly (a multiple of 2^-s in
-    //   [-1, 1)): floor(a b / 2^s) = f + floor(fma(a, bs, -f)).
-    // No compare or branch: the chain stays on the vector unit.  A fixed
-    // point stays fixed, and so does 1 (the reference's value once a step
-    // gives y <= 0), so running every remaining step gives the reference's
-    // y.  Should y ever reach 2^49 the integer steps below run instead.
+    // Steps 1..7 on exact doubles, FP64 rounding down (q48_round_down):
+    // with M = 1.5 2^52 and xs = xn 2^-48,
+    //   t1 = fma(y, y 2^-48, M)      = M + y2,  y2 = floor(y^2 / 2^48)
+    //   t2 = fma(t1, xs, M - M xs)   = M + xy2, xy2 = floor(xn y2 / 2^48)
+    //   fs = fma(t2, -2^-49, ...)    = (3 2^48 - xy2) 2^-49, exact
+    //   t3 = fma(y, fs, M)           = M + the next y
+    // (M xs is a multiple of 24 below 2^55 and M - M xs one of 8 below 2^54:
+    // both exact), each truncated product one operation while its value
+    // stays within 2^51 of 0.  xn < 2^50, so that holds while 1 <= y < 2^49
+    // (y2 <= 2^50; xy2 near 2^48 as y nears 1 / sqrt(xn)); a value past
+    // those bounds rounds to a coarser grid but stays past them, so the
+    // largest and smallest y tell, and the integer steps below run instead.
+    // They also hold the reference's clamp of y <= 0 to 1, which xn in [2^48,
+    // 2^50) never reaches (80 million arguments checked on the host).  The
+    // chain is five dependent operations a step; rounding to nearest took 18.
     if (i < 8) {
+        const double M = 0x1.8p52;
         const double xs = (double)xn * 0x1p-48;                 // exact
-        const double tq = 844424930131968.0 * 0x1p-49;          // 3 * 2^48 * 2^-49
-        double yd = (double)y, mx = yd;
+        const double cx = __builtin_fma(-M, xs, M);             // exact
+        const double tq = (844424930131968.0 + M) * 0x1p-49;    // (3 2^48 + M) 2^-49
+        double yd = (double)y, ys = yd * 0x1p-48, mx = yd, mn = yd;
 #pragma unroll
         for (int j = 0; j < 7; ++j) {
-            const double ys = yd * 0x1p-48;
-            double P = yd * ys, f = __builtin_floor(P);
-            const double y2 = f + __builtin_floor(__fma_rn(yd, ys, -f));
-            P = y2 * xs;
-            f = __builtin_floor(P);
-            const double xy2 = f + __builtin_floor(__fma_rn(y2, xs, -f));
-            const double fs = __fma_rn(xy2, -0x1p-49, tq);     // (3 * 2^48 - xy2) 2^-49
-            P = yd * fs;
-            f = __builtin_floor(P);
-            yd = __builtin_fmax(f + __builtin_floor(__fma_rn(yd, fs, -f)), 1.0);
+            const double t1 = __builtin_fma(yd, ys, M);
+            const double t2 = __builtin_fma(t1, xs, cx);
+            const double fs = __builtin_fma(t2, -0x1p-49, tq);
+            const double t3 = __builtin_fma(yd, fs, M);
+            yd = t3 - M;
+            ys = __builtin_fma(t3, 0x1p-48, -M * 0x1p-48);
             mx = __builtin_fmax(mx, yd);
+            mn = __builtin_fmin(mn, yd);
         }
-        if (mx < 562949953421312.0) {   // 2^49
+        if (mx < 562949953421312.0 && mn >= 1.0) {   // 2^49
             y = (int64_t)yd;
             i = 8;
         }
@@ -542,27 +564,25 @@ __device__ __forceinline__ int64_t q48_exp(int64_t x)
 }
 
 // fp_exp for |x| <= 10 ONE, the range fp_safe_exp leaves (fp_math.h:739-744):
-// the same squarings, the first 12 on exact doubles.  r0 = ONE + (|x| >> 14)
-// and r_k = floor(r_{k-1}^2 / 2^48) <= e^(10 2^(k - 14)) ONE, so r_0 .. r_11
-// stay below 3.5 ONE < 2^50, each of their squares is below 2^100 and r_12 is
-// below 12.2 ONE < 2^52: with rs = r 2^-48 (exact), f = floor(r rs) and
-// fma(r, rs, -f) = (r^2 - f 2^48) 2^-48 exactly (a multiple of 2^-48 in [-1,
-// 1)), floor(r^2 / 2^48) = f + floor(fma(r, rs, -f)), an integer double.
-// Full-rate FP64 instead of three quarter-rate 32 x 32 -> 64 products per
-// square; the last two squares (up to e^10 ONE < 2^63) stay integer, and the
-// reciprocal of a negative argument is q48_recip (r >= ONE).
+// the same squarings, the first 12 on exact doubles, FP64 rounding down
+// (q48_round_down).  r0 = ONE + (|x| >> 14) and r_k = floor(r_{k-1}^2 / 2^48)
+// <= e^(10 2^(k - 14)) ONE, so r_12 stays below 12.2 ONE < 2^52: with y = r
+// 2^-24, h = fma(y, y, 2^52) is 2^52 + r_k exactly and fma(h, 2^-24, -2^28) the
+// next y, two dependent operations a square (eight with rounding to nearest;
+// three quarter-rate 32 x 32 -> 64 products on integers).  The last two
+// squares (up to e^10 ONE < 2^63) stay integer, and the reciprocal of a
+// negative argument is q48_recip (r >= ONE).
 __device__ __forceinline__ int64_t q48_exp_small(int64_t x)
 {
     const uint64_t m = x >= 0 ? (uint64_t)x : (uint64_t)0 - (uint64_t)x;
-    double rd = (double)(int64_t)((uint64_t)Q48_ONE + (m >> 14));
+    // r0 < 2^52: its double from the word of r0 + 2^52
+    double h = __builtin_bit_cast(double, 0x4330000000000000ull + (uint64_t)Q48_ONE + (m >> 14));
 #pragma unroll
     for (int k = 0; k < 12; ++k) {
-        const double rs = rd * 0x1p-48;
-        const double f = __builtin_floor(rd * rs);
-        rd = f + __builtin_floor(__fma_rn(rd, rs, -f));
+        const double y = __builtin_fma(h, 0x1p-24, -0x1p28);
+        h = __builtin_fma(y, y, 0x1p52);
     }
-    // rd is an integer below 2^52: the low bits of rd + 2^52's word
-    uint64_t u = (uint64_t)__builtin_bit_cast(int64_t, rd + 0x1p52) - 0x4330000000000000ull;
+    uint64_t u = q48_word_m52(h);
     u = (uint64_t)q48_usqr(u);
     u = (uint64_t)q48_usqr(u);
     if (x > 0)

@@ -228,6 +228,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
                                                     int *__restrict__ rms_count,
                                                     int M, int K, int seg, const q48_ropekv rk)
 {
+    q48_round_down();
     extern __shared__ __align__(16) uint32_t xs[];   // 3 limbs per staged x
     __shared__ uint64_t red_lo[NW], red_hi[NW];
     __shared__ uint64_t part[NW][V4_RB][2];
@@ -683,6 +684,7 @@ __global__ __launch_bounds__(64 * RW) void k_gemv_r1(int64_t *__restrict__ y,
                                                      const int64_t *__restrict__ r_in, int M,
                                                      const q48_ropekv rk)
 {
+    q48_round_down();
     static_assert(RW % 2 == 0 && NT % UNR == 0, "row pairs, whole windows");
     constexpr int TE = WFmt<WT>::TE * 8;                // elements per 1 KB tile
     constexpr int K = TE * NT;
@@ -893,6 +895,7 @@ k_gemv_p6(int64_t *__restrict__ y, const void *__restrict__ Wv,
           const int64_t *__restrict__ x, const int64_t *__restrict__ norm_w,
           const int64_t *__restrict__ r_in, int M, int K, int seg)
 {
+    q48_round_down();
     static_assert(NTF > 0 && (PRO == 0 || PRO == 3) && (EPI == 0 || EPI == 2), "p6 forms");
     // the window crosses into the next group in the slots it frees: tile t of
     // the next group must land in slot t % UNR
@@ -1086,6 +1089,7 @@ __global__ __launch_bounds__(256) void k_rms_inv(int64_t *__restrict__ r_out,
                                                 const int *__restrict__ d_token, int token,
                                                 int dim)
 {
+    q48_round_down();
     __shared__ uint64_t red_lo[4], red_hi[4];
     const int tid = threadIdx.x;
     if (table) {
@@ -1165,6 +1169,7 @@ __global__ __launch_bounds__(256) void k_rms_stats(int64_t *__restrict__ stats,
 __global__ __launch_bounds__(256) void k_stats_r(int64_t *__restrict__ r_out,
                                                 const int64_t *__restrict__ stats, int dim)
 {
+    q48_round_down();
     __shared__ uint64_t red_lo[4], red_hi[4];
     const int np = (dim + 7) >> 3;
     const uint64_t *st = reinterpret_cast<const uint64_t *>(stats);

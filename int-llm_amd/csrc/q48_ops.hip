@@ -32,6 +32,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm(int64_t *__restrict__ out,
                                                 const int64_t *__restrict__ w,
                                                 int dim)
 {
+    q48_round_down();
     __shared__ uint64_t red_lo[4], red_hi[4];
     __shared__ int64_t r_sh;
     const int tid = threadIdx.x;
@@ -82,8 +83,10 @@ __global__ __launch_bounds__(256) void k_rope_init(int64_t *__restrict__ cos_t,
     q48_sincos(k, q48_mul(q48_from_int(pos), th), &c, &s);
     cos_t[idx] = c;
     sin_t[idx] = s;
-    if (idx == 0)   // the attention score scale, stored after the sine table
+    if (idx == 0) {   // the attention score scale, stored after the sine table
+        q48_round_down();
         sin_t[(size_t)half * max_seq] = q48_inv_sqrt(q48_from_int(head_dim));
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -130,6 +133,7 @@ __global__ __launch_bounds__(ATT_NT) void k_attn_decode(
     int64_t *__restrict__ scores, int layer, const int *__restrict__ d_pos, int pos,
     int n_heads, int n_kv, int hd, int max_seq)
 {
+    q48_round_down();
     __shared__ int64_t qs[256];
     __shared__ int64_t red[ATT_NT / 64];
     __shared__ int64_t part[ATT_NT];
@@ -229,6 +233,7 @@ __global__ __launch_bounds__(ATT_NT) void k_attn_v2(
     int n_heads, int n_kv, int hd, int max_seq, const ulonglong2 *__restrict__ pf,
     size_t pf_n16)
 {
+    q48_round_down();
     __shared__ int64_t qs[256], ks[256], vs[256];
     __shared__ int64_t red[ATT_NT / 64];
     __shared__ int64_t part[ATT_NT];
@@ -382,6 +387,7 @@ __global__ __launch_bounds__(NT) void k_attn_v3(
     const int *__restrict__ d_pos, int pos, int n_heads, int n_kv, int max_seq,
     const ulonglong2 *__restrict__ pf, size_t pf_n16)
 {
+    q48_round_down();
     if ((int)blockIdx.x >= n_heads) {
         const size_t stride = (size_t)(gridDim.x - n_heads) * NT;
         size_t i = (size_t)(blockIdx.x - n_heads) * NT + threadIdx.x;
@@ -579,6 +585,7 @@ __global__ __launch_bounds__(256) void k_attn_se(int64_t *__restrict__ out,
                                                 const int *__restrict__ d_pos, int pos,
                                                 int n_heads, int max_seq)
 {
+    q48_round_down();
     constexpr int NT = 256;
     static_assert(ATT_CH == NT, "one position per thread");
     __shared__ int64_t red[NT / 64];
@@ -615,6 +622,7 @@ __global__ __launch_bounds__(256) void k_attn_s2(int64_t *__restrict__ out,
                                                 const int *__restrict__ d_pos, int pos,
                                                 int n_heads, int n_kv, int max_seq)
 {
+    q48_round_down();
     constexpr int NT = 256, SL = NT / HD, VB = 8;
     __shared__ int64_t part[NT], pl[ATT_CH], red[NT / 64];
     if (d_pos)
@@ -846,6 +854,7 @@ __global__ __launch_bounds__(ATTG_NT) __attribute__((amdgpu_waves_per_eu(HD == 1
     uint64_t *__restrict__ xbuf, int layer, const int *__restrict__ d_pos, int pos,
     int n_heads, int n_kv, int max_seq, uint64_t tmo)
 {
+    q48_round_down();
     constexpr int NT = ATTG_NT, CH = ATTG_CH, GM = ATTG_GMAX;
     constexpr int HALF = HD / 2, RS = HD + 1;
     constexpr int RP = (GM * HALF + NT - 1) / NT;       // RoPE pairs per thread
@@ -1352,6 +1361,7 @@ __global__ __launch_bounds__(256) void k_step_record(const int *__restrict__ st,
 __global__ __launch_bounds__(256) void k_silu_mul_pairs(int64_t *__restrict__ out,
                                                        const int64_t *__restrict__ t, int n)
 {
+    q48_round_down();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n)
         out[i] = q48_mul(q48_silu(t[2 * i]), t[2 * i + 1]);
@@ -1362,6 +1372,7 @@ __global__ __launch_bounds__(256) void k_silu_mul(int64_t *__restrict__ out,
                                                  const int64_t *__restrict__ g,
                                                  const int64_t *__restrict__ u, int n)
 {
+    q48_round_down();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n)
         out[i] = q48_mul(q48_silu(g[i]), u[i]);
@@ -1447,6 +1458,9 @@ __global__ __launch_bounds__(256) void k_fp_eval(int func, const int64_t *__rest
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n)
         return;
+    // the functions written for rounding down; the others keep the default
+    if (func == 4 || (func >= 8 && func <= 10) || func == 12)
+        q48_round_down();
     const int64_t a = x[i];
     int64_t r = 0, r1 = 0;
     switch (func) {

@@ -160,6 +160,7 @@ k_pfa(int64_t *__restrict__ out,
                                             const int64_t *__restrict__ scale_p, int p0, int T,
                                             int n_heads, int n_kv, int Ppad, size_t per_head)
 {
+    q48_round_down();
     constexpr int HDP = HD < 64 ? 64 : HD, KS = HDP / 64;
     constexpr int NDT = HD / 16, DTW = (NDT + 3) / 4;   // 16-dim tiles, per wave
     constexpr int DB = HD / 4, JG = 64 / DB, JPER = PF_STEP / JG;

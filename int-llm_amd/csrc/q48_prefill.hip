@@ -62,6 +62,7 @@ __global__ __launch_bounds__(256) void k_pf_attn(int64_t *__restrict__ out,
                                                 const int64_t *__restrict__ scale_p, int layer,
                                                 int p0, int n_heads, int n_kv, int max_seq)
 {
+    q48_round_down();
     const int t = blockIdx.y;
     const size_t row = (size_t)(n_heads + 2 * n_kv) * HD;
     attn_v3_head<HD, ATT_LDS_MAX, false, true>(
@@ -75,6 +76,7 @@ __global__ __launch_bounds__(256) void k_pf_attn(int64_t *__restrict__ out,
 __global__ __launch_bounds__(256) void k_pf_silu(int64_t *__restrict__ out,
                                                 const int64_t *__restrict__ GU, int ffn)
 {
+    q48_round_down();
     const int t = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
     if (i < ffn) {
         const int64_t *g = GU + (size_t)t * 2 * ffn;

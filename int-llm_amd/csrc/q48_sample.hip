@@ -365,6 +365,7 @@ __global__ __launch_bounds__(SMP_B) void k_smp_topk(int64_t *__restrict__ base, 
 // ---- 3: e = fp_safe_exp(x - max) (softmax, llama_int.c:1060-1072) --------
 __global__ __launch_bounds__(SMP_T) void k_smp_exp(int64_t *__restrict__ base, int n)
 {
+    q48_round_down();
     __shared__ int64_t red[SMP_T / 64];
     SmpWs s = smp_ws(base, n);
     const int64_t thr = s.st[ST_THR], mx = s.st[ST_MX];
@@ -399,6 +400,7 @@ __device__ __forceinline__ q48_u128 smp_total(const SmpWs &s, int nblk)
 // ---- 4: p = fp_div(e, sum) when sum > 0 -----------------------------------
 __global__ __launch_bounds__(SMP_T) void k_smp_div(int64_t *__restrict__ base, int n, int nblk)
 {
+    q48_round_down();
     __shared__ int64_t sum_sh;
     SmpWs s = smp_ws(base, n);
     if (threadIdx.x == 0) {
@@ -503,6 +505,7 @@ __global__ __launch_bounds__(SMP_B) void k_smp_pick(int64_t *__restrict__ base, 
                                                    int *__restrict__ st, int *__restrict__ tokens,
                                                    int cap)
 {
+    q48_round_down();
     __shared__ int64_t redv[SMP_B / 64];
     __shared__ int redi[SMP_B / 64];
     __shared__ uint64_t scan[SMP_B / 64];
