@@ -87,6 +87,11 @@ __device__ __forceinline__ void attn_v3_head(
     __shared__ int64_t red[NT / 64], red2[NT / 64];
     __shared__ int64_t part[NT];
     __shared__ int64_t sc[SMAX];
+    __shared__ int form, big_v;   // set by any thread that sees the case, below
+    if (threadIdx.x == 0) {
+        form = 0;
+        big_v = 0;
+    }
     if (!ROT) {
         if (d_pos)
             pos = *d_pos;
@@ -246,26 +251,70 @@ __device__ __forceinline__ void attn_v3_head(
     // slot writes (the one after them also orders the score stores)
     mx = block_max64<NT>(mx, red, false);
     int64_t sum = 0;
+    int odd = 0;
     for (int t = tid; t < S; t += NT) {
         const int64_t e = q48_safe_exp((int64_t)((uint64_t)sc[t] - (uint64_t)mx));
         sc[t] = e;
         sum = (int64_t)((uint64_t)sum + (uint64_t)e);
+        odd |= (uint64_t)e > (uint64_t)Q48_ONE ? 1 : 0;
     }
     sum = block_sum64<NT>(sum, red2, false);
-    // the weights are never negative (exponentials over a positive sum, or
-    // the exponentials themselves); checked, and the values take the product
-    // for non-negative weights (q48_pv_mac) unless one is
-    int neg = 0;
+    // The weights' form, chosen once for the block: with every exponential in
+    // [0, ONE] their sum is exact and positive and the weights add up to at
+    // most ONE, so the values take one FP64 operation per term (q48_fsum8);
+    // wrapped score differences may give larger ones (bit 0: any), and then
+    // the weights are either all non-negative (q48_pv_mac) or not (bit 1).
     const q48_divisor dv = q48_divisor_of(sum);
     for (int t = tid; t < S; t += NT) {
         if (sum > 0)
             sc[t] = q48_div_by(sc[t], dv);
-        neg |= sc[t] < 0;
+        odd |= sc[t] < 0 ? 3 : 0;
     }
-    neg = __syncthreads_or(neg);
+    if (odd)
+        atomicOr(&form, odd);
+    __syncthreads();
+    const int wide = form & 1, neg = form & 2;
 
-    // o[d] = sum_t fp_mul(p_t, v_t[d]), llama_int.c:1514-1529; one copy of
-    // the loop per product form, chosen once for the block
+    // o[d] = sum_t fp_mul(p_t, v_t[d]), llama_int.c:1514-1529.  The FP64 sums:
+    // lane l of a row of 16 holds the weight of its slice's position i0 + l
+    // % 16 (0 past S).  17 VALU operations and an LDS read per term became
+    // about five operations and no read: 9.5 -> 8.5 us a call at 121 positions.
+    double facc = Q48_FSUM0;
+    uint32_t big = 0;
+    if (!wide) {
+        auto fmac = [&](auto base, const int64_t(&vv)[VB], int i0, double p) {
+            double f[VB];
+#pragma unroll
+            for (int u = 0; u < VB; ++u)
+                f[u] = q48_f51(!ROT && sl + SL * (i0 + u) == pos ? vs[d] : vv[u], big);
+            q48_fsum8<decltype(base)::value>(facc, p, f);
+        };
+        for (int i0 = 0; sl + SL * i0 < S; i0 += 2 * VB) {
+            const int tp = sl + SL * (i0 + (tid & 15));
+            const double p = tp < S ? q48_pscaled(sc[tp]) : 0.0;
+            fmac(std::integral_constant<int, 0>{}, va, i0, p);
+            if (SL * (i0 + 2 * VB) < S) {
+#pragma unroll
+                for (int u = 0; u < VB; ++u)
+                    va[u] = vld(i0 + 2 * VB + u);
+            }
+            if (SL * (i0 + VB) < S)
+                fmac(std::integral_constant<int, VB>{}, vb, i0 + VB, p);
+            if (SL * (i0 + 3 * VB) < S) {
+#pragma unroll
+                for (int u = 0; u < VB; ++u)
+                    vb[u] = vld(i0 + 3 * VB + u);
+            }
+        }
+    }
+    part[tid] = q48_fsum_total(facc);
+    if (q48_f51_big(big))
+        big_v = 1;
+    __syncthreads();
+    const bool over = wide || big_v;
+
+    // the general products, where a weight or a value is out of that range;
+    // one copy of the loop per product form
     auto values = [&](auto nonneg) -> uint64_t {
         uint64_t acc = 0;
         q48_pv_acc pa = {0, 0};
@@ -282,6 +331,12 @@ __device__ __forceinline__ void attn_v3_head(
                 }
             }
         };
+#pragma unroll
+        for (int u = 0; u < VB; ++u)
+            va[u] = vld(u);
+#pragma unroll
+        for (int u = 0; u < VB; ++u)
+            vb[u] = vld(VB + u);
         for (int i0 = 0; sl + SL * i0 < S; i0 += 2 * VB) {
             // the next batches where some position of them exists (as above)
             vmac(va, i0);
@@ -300,9 +355,10 @@ __device__ __forceinline__ void attn_v3_head(
         }
         return acc + (uint64_t)q48_pv_total(pa);
     };
-    const uint64_t acc = neg ? values(std::false_type{}) : values(std::true_type{});
-    part[tid] = (int64_t)acc;
-    __syncthreads();
+    if (over) {   // uniform over the block
+        part[tid] = (int64_t)(neg ? values(std::false_type{}) : values(std::true_type{}));
+        __syncthreads();
+    }
     if (sl == 0) {
         uint64_t o = 0;
 #pragma unroll

@@ -265,6 +265,64 @@ __device__ __forceinline__ int64_t q48_pv_total(const q48_pv_acc &acc)
     return (int64_t)(acc.a1 + (acc.a2 << 16));
 }
 
+// The same sums on FP64 rounding down (q48_round_down), one fused operation
+// per term: with p_t' = p_t 2^-48 (exact) and |v_t| < 2^51, fma(p_t', v_t, acc)
+// adds floor(p_t v_t / 2^48) exactly to an accumulator that starts at
+// Q48_FSUM0 = 1.5 2^52 and stays in [2^52, 2^53), where doubles are the
+// integers.  It stays there while 0 <= p_t <= ONE and sum p_t <= ONE: each
+// partial sum is within (sum p_t) 2^51 / 2^48 = 2^51 of the start.  A softmax
+// row gives that whenever every exponential is at most ONE (no wrapped score
+// difference), since fp_div truncates; callers check both conditions on the
+// data and take q48_pv_mac (or q48_mul) otherwise.
+#define Q48_FSUM0 0x1.8p52
+
+// v as a double (|v| < 2^51: the word of v + 1.5 2^52 is v's plus a constant
+// in the high half); big collects high-word bits that tell whether any v was
+// outside that range (q48_f51_big).
+__device__ __forceinline__ double q48_f51(int64_t v, uint32_t &big)
+{
+    const uint32_t hi = (uint32_t)((uint64_t)v >> 32);
+    big |= hi + 0x80000u;
+    return __builtin_bit_cast(double, ((uint64_t)(hi + 0x43380000u) << 32) | (uint32_t)v) -
+           Q48_FSUM0;
+}
+__device__ __forceinline__ bool q48_f51_big(uint32_t big) { return (big & 0xFFF00000u) != 0; }
+
+// p 2^-48 for 0 <= p <= ONE
+__device__ __forceinline__ double q48_pscaled(int64_t p)
+{
+    return __builtin_fma(__builtin_bit_cast(double, (uint64_t)p | 0x4330000000000000ull),
+                         0x1p-48, -16.0);
+}
+
+__device__ __forceinline__ int64_t q48_fsum_total(double acc)
+{
+    return __builtin_bit_cast(int64_t, acc) - __builtin_bit_cast(int64_t, Q48_FSUM0);
+}
+
+// acc += the eight terms p[BASE + n] v[n]: lane BASE + n of every row of 16
+// lanes holds its row's weight for v[n] (row_newbcast gives it to the row),
+// so one register pair carries 16 weights and none comes from LDS per term.
+// The s_nop covers the wait states between a vector write of p and its DPP
+// read.  Every lane of a row must be active or none.
+template <int BASE>
+__device__ __forceinline__ void q48_fsum8(double &acc, double p, const double (&v)[8])
+{
+    asm("s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %3 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %4 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %5 row_newbcast:%13 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %6 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %7 row_newbcast:%15 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %8 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %9 row_newbcast:%17 row_mask:0xf bank_mask:0xf"
+        : "+v"(acc)
+        : "v"(p), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]),
+          "v"(v[7]), "n"(BASE), "n"(BASE + 1), "n"(BASE + 2), "n"(BASE + 3), "n"(BASE + 4),
+          "n"(BASE + 5), "n"(BASE + 6), "n"(BASE + 7));
+}
+
 // fp_mul(r, r): r * r = u^2 with u = |r| <= 2^63 as an unsigned word;
 // u^2 = hh 2^64 + 2 lh 2^32 + ll, and w = 2 lh + (ll >> 32) stays below 2^64,
 // so bits 48..111 are (hh << 16) + (w >> 16) mod 2^64: three 32 x 32 -> 64

@@ -872,6 +872,10 @@ __global__ __launch_bounds__(ATTG_NT) __attribute__((amdgpu_waves_per_eu(HD == 1
     __shared__ int64_t sc[GM][CH];
     __shared__ q48_u128 dpart[MF ? 1 : GM * CH];
     __shared__ int64_t loc[GM];
+    __shared__ uint64_t csum[GM];                        // the chunk's sums
+    __shared__ int form;                                 // of the value products
+    if (threadIdx.x == 0)
+        form = 0;
     // the exchange buffer, and before it the key digit planes (MF)
     __shared__ union __align__(16) {
         int64_t got[GM][ATTG_NCMAX];
@@ -966,6 +970,22 @@ __global__ __launch_bounds__(ATTG_NT) __attribute__((amdgpu_waves_per_eu(HD == 1
         kl[rr][rw + 2 * d + 1] = (int64_t)kr[d].y;
         vl[rr][rw + 2 * d] = (int64_t)vr[d].x;
         vl[rr][rw + 2 * d + 1] = (int64_t)vr[d].y;
+    }
+    // 1: a value outside q48_fsum8's range, or (below) an exponential above
+    // ONE; the staged rows count, and the new value (the row at pos, staged
+    // from the cache, is replaced by it: what was there before may only make
+    // the block take the general products)
+    int wide;
+    {
+        uint32_t big = 0;
+#pragma unroll
+        for (int d = 0; d < LW / 2; ++d) {
+            big |= (uint32_t)(vr[d].x >> 32) + 0x80000u;
+            big |= (uint32_t)(vr[d].y >> 32) + 0x80000u;
+        }
+        if (pos < tend)
+            big |= (uint32_t)((uint64_t)vn >> 32) + 0x80000u;
+        wide = q48_f51_big(big) ? 1 : 0;
     }
     __syncthreads();
     if (pos < tend && tid < HD) {   // the row at pos: this block's rotated k, new v
@@ -1086,7 +1106,8 @@ __global__ __launch_bounds__(ATTG_NT) __attribute__((amdgpu_waves_per_eu(HD == 1
         q48_u128 dot = 0;
         if (hh < G) {
             const int64_t *qa = qs[hh] + dh * DH, *ka = kl[t] + dh * DH;
-#pragma unroll 8
+            constexpr int UD = HD == 64 ? 4 : 8;   // 8 spills at head_dim 64
+#pragma unroll UD
             for (int d = 0; d < DH; ++d)
                 dot += (q48_u128)q48_smul128(qa[d], ka[d]);
         }
@@ -1128,14 +1149,20 @@ __global__ __launch_bounds__(ATTG_NT) __attribute__((amdgpu_waves_per_eu(HD == 1
     }
 
     // e_t = fp_safe_exp(s_t - max), one per thread, and the chunk sums
-    if (dh == 0 && hh < G)
-        sc[hh][t] = live ? q48_safe_exp((int64_t)((uint64_t)sc[hh][t] - (uint64_t)loc[hh])) : 0;
+    if (dh == 0 && hh < G) {
+        const int64_t e =
+            live ? q48_safe_exp((int64_t)((uint64_t)sc[hh][t] - (uint64_t)loc[hh])) : 0;
+        sc[hh][t] = e;
+        wide |= (uint64_t)e > (uint64_t)Q48_ONE ? 1 : 0;
+    }
     __syncthreads();
     if (tid < 32 * GM) {
         const int hq = tid >> 5, u = tid & 31;
         const uint64_t sm = attg_sum32(hq < G && u < nt ? (uint64_t)sc[hq][u] : 0);
-        if (u == 0 && hq < G)
+        if (u == 0 && hq < G) {
             loc[hq] = (int64_t)sm;
+            csum[hq] = sm;
+        }
     }
     __syncthreads();
     if (nc > 1) {
@@ -1157,28 +1184,56 @@ __global__ __launch_bounds__(ATTG_NT) __attribute__((amdgpu_waves_per_eu(HD == 1
             __hip_atomic_store(ep, E + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
     }
-    // p_t = fp_div(e_t, sum) when sum > 0 (llama_int.c:1069-1071).  The
-    // weights are never negative (exponentials over a positive sum, or the
-    // exponentials themselves); the block checks it, and the values take
-    // the product for non-negative weights (q48_pv_mac) unless one is
-    int neg = 0;
+    // p_t = fp_div(e_t, sum) when sum > 0 (llama_int.c:1069-1071).  The form
+    // of the value products, chosen for the block: FP64 sums (q48_fsum8)
+    // when its exponentials are in [0, ONE], its share of the sum is at most
+    // the sum (so its weights add up to at most ONE) and its values are below
+    // 2^51; otherwise q48_pv_mac while no weight is negative (weights are
+    // exponentials over a positive sum, or the exponentials themselves), or
+    // q48_mul (bit 1).
+    int odd = wide;
     if (dh == 0 && live) {
         const int64_t sum = loc[hh];
         if (sum > 0)
             sc[hh][t] = q48_div_by(sc[hh][t], q48_divisor_of(sum));
-        neg = sc[hh][t] < 0;
+        odd |= sc[hh][t] < 0 ? 3 : sum <= 0 || csum[hh] > (uint64_t)sum ? 1 : 0;
     }
-    neg = __syncthreads_or(neg);
+    if (odd)
+        atomicOr(&form, odd);
+    __syncthreads();
+    const int gen = form & 1, neg = form & 2;
 
     // o[h][d] += sum_t fp_mul(p_t, v_t[d]) over the chunk: thread owns the
-    // outputs tid + NT o of the group's [G][HD]
+    // outputs tid + NT o of the group's [G][HD], so that a row of 16 lanes
+    // shares a head: two register pairs a lane carry the head's 32 weights
+    // (0 past the chunk's last position), and a term is one LDS read of the
+    // value, its conversion and one FP64 operation, where two LDS reads and 17
+    // operations took 2.9 us of a block's 16.5 (16.0 -> 14.1 us a call at 2061
+    // positions).
 #pragma unroll
     for (int o = 0; o < NO; ++o) {
         const int oi = tid + o * NT;
         if (oi < G * HD) {
             const int oh = oi / HD, d = oi % HD;
             uint64_t acc = 0;
-            if (!neg) {
+            if (!gen) {
+                double fa = Q48_FSUM0;
+                uint32_t none = 0;
+#pragma unroll
+                for (int g = 0; g < CH; g += 16) {
+                    const double p = q48_pscaled(sc[oh][g + (tid & 15)]);
+                    double f[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        f[u] = q48_f51(vl[g + u][d], none);
+                    q48_fsum8<0>(fa, p, f);
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        f[u] = q48_f51(vl[g + 8 + u][d], none);
+                    q48_fsum8<8>(fa, p, f);
+                }
+                acc = (uint64_t)q48_fsum_total(fa);
+            } else if (!neg) {
                 q48_pv_acc pa = {0, 0};
                 for (int u = 0; u < nt; ++u)
                     q48_pv_mac(pa, sc[oh][u], vl[u][d]);
