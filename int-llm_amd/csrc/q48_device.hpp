@@ -323,6 +323,25 @@ __device__ __forceinline__ void q48_fsum8(double &acc, double p, const double (&
           "n"(BASE + 5), "n"(BASE + 6), "n"(BASE + 7));
 }
 
+// Four positions of four rows: acc[r] += p[r][BASE + n] v[n], the rows in
+// turn, so that each sum's next term is three others away.
+template <int BASE>
+__device__ __forceinline__ void q48_fsum4x4(double &a0, double &a1, double &a2, double &a3,
+                                            const double (&p)[4], const double (&v)[4])
+{
+#define Q48_FS4(V, N)                                                            \
+    "v_fmac_f64_dpp %0, %4, %" V " row_newbcast:%" N " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f64_dpp %1, %5, %" V " row_newbcast:%" N " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f64_dpp %2, %6, %" V " row_newbcast:%" N " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f64_dpp %3, %7, %" V " row_newbcast:%" N " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" Q48_FS4("8", "12") Q48_FS4("9", "13") Q48_FS4("10", "14")
+            Q48_FS4("11", "15")
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3)
+        : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]),
+          "n"(BASE), "n"(BASE + 1), "n"(BASE + 2), "n"(BASE + 3));
+#undef Q48_FS4
+}
+
 // fp_mul(r, r): r * r = u^2 with u = |r| <= 2^63 as an unsigned word;
 // u^2 = hh 2^64 + 2 lh 2^32 + ll, and w = 2 lh + (ll >> 32) stays below 2^64,
 // so bits 48..111 are (hh << 16) + (w >> 16) mod 2^64: three 32 x 32 -> 64

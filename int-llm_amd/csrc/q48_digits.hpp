@@ -1,6 +1,5 @@
 // q48_digits.hpp — int64 values as eight int8 digits for the int8 matrix
-// cores, and the 24-bit limb products of truncated Q16.48 products.  Included
-// by the HIP sources of libintllm_hip only.
+// cores.  Included by the HIP sources of libintllm_hip only.
 //
 // Digits.  Every int64 v is written v = S(v) + C with C = 0x0080808080808080
 // and S(v) = sum_i s_i 256^i, s_i the bytes of v ^ C read as int8 (bytes 0..6
@@ -134,36 +133,6 @@ __device__ __forceinline__ q48_u128 digits_total14(const int (&a)[14])
     for (int g = 2; g >= 0; --g)
         tot = (tot << 32) + (q48_u128)(q48_i128)part[g];
     return tot;
-}
-
-// v_mad_u32_u24: a * b + c over the low 24 bits of a and b (full rate)
-__device__ __forceinline__ uint32_t mad_u24(uint32_t a, uint32_t b, uint32_t c)
-{
-    uint32_t r;
-    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-
-// Low limbs of a truncated product.  For a = p mod 2^48 = a0 + 2^24 a1 and
-// b = v mod 2^48 = b0 + 2^24 b1 (24-bit limbs; a limb word may carry higher
-// bits, the 24-bit multiplies ignore them), t = floor(((p v) mod 2^48) / 2^24)
-//   = (a0 b1 + a1 b0 + floor(a0 b0 / 2^24)) mod 2^24;
-// returns acc + t.  Then for any n terms (n < 2^24)
-//   sum_j floor(p_j v_j / 2^48) = floor((sum_j p_j v_j - 2^24 sum_j t_j) / 2^48),
-// since each (p_j v_j) mod 2^48 lies in [2^24 t_j, 2^24 t_j + 2^24).
-__device__ __forceinline__ uint32_t trunc_low_acc(uint2 a, uint2 b, uint32_t acc)
-{
-    const uint64_t p00 = (uint64_t)(a.x & 0xFFFFFFu) * (b.x & 0xFFFFFFu);
-    uint32_t t = __builtin_amdgcn_alignbit((uint32_t)(p00 >> 32), (uint32_t)p00, 24);
-    t = mad_u24(a.x, b.y, t);
-    t = mad_u24(a.y, b.x, t);
-    return mad_u24(t, 1u, acc);
-}
-
-// the limb words (bits 0..31, bits 24..55) of v for trunc_low_acc
-__device__ __forceinline__ uint2 low_limbs(uint64_t v)
-{
-    return make_uint2((uint32_t)v, __builtin_amdgcn_alignbit((uint32_t)(v >> 32), (uint32_t)v, 24));
 }
 
 } // namespace

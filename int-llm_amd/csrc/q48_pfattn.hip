@@ -8,11 +8,13 @@
 //   v_mfma_i32_16x16x64_i8 per 16 x 16 tile and 64 dims.
 // Weights.  The softmax on the VALU: exact maximum, fp_safe_exp of the
 //   wrapped difference, wrapping sum, fp_div when the sum is positive.
-// Values.  o_d = sum_j fp_mul(p_j, v_j,d) truncates every product.  With
-//   X_d = sum_j p_j v_j,d from the digit identity over j and Λ_d = sum_j t_j,d
-//   the 24-bit limb term of trunc_low_acc, o_d = (X_d - 2^24 Λ_d) >> 48: the
-//   MFMA digit products plus six full-rate VALU instructions per (row,
-//   position, dim) instead of a 64 x 64 -> 128 product each.
+// Values.  o_d = sum_j fp_mul(p_j, v_j,d) truncates every product: one FP64
+//   operation per (row, position, dim), rounding down (q48_fsum4x4), for
+//   values in [-2^51, 2^51).  A block whose span holds a larger value splits
+//   v = v1 + 2^48 v2 (v1 = v mod 2^48) and the weight p = pa + 2^24 pb, and
+//   makes three such sums, o = sum floor(p v1 / 2^48) + sum pa v2 + 2^24 sum
+//   pb v2, the last two exact integers below 2^51; one whose weights are not
+//   a plain softmax (wrapped score differences) multiplies in integers.
 //
 // A block owns 16 consecutive query rows of one head.  k_pfa_prep first
 // writes the layer's keys and values as digit planes once per KV head; the
@@ -60,22 +62,19 @@ __device__ __forceinline__ void st128(uint64_t *p, q48_u128 v)
     p[1] = (uint64_t)(v >> 64);
 }
 
-// Digit planes of the layer's keys and values at positions [64 c, 64 c + 64)
-// of KV head kh (grid (Ppad / 64, n_kv)); positions at or past P read as C
-// (all digits zero):
+// Digit planes of the layer's keys, and its values as doubles, at positions
+// [64 c, 64 c + 64) of KV head kh (grid (Ppad / 64, n_kv)); keys at or past P
+// read as C (all digits zero), values as 0:
 //  KD[kh][a][j][HDP]   digit a of k_j,d (HDP: head_dim rounded up to 64, the
 //                      pad dims zero digits)
-//  VD[kh][a][d][Ppad]  digit a of v_j,d
-//  CK[kh][j]           C sum_d k_j,d - hd C^2
-//  VS[kh][c][d]        sum of v_j,d over the 64 positions of c
-//  VL[kh][j][d]        low_limbs(v_j,d) (0 past P)
-// (int128 values as two words, low first).
+//  CK[kh][j]           C sum_d k_j,d - hd C^2 (int128, low word first)
+//  VF[kh][j][d]        v_j,d (where it is within [-2^51, 2^51))
+//  VB[kh][c]           1 when some v of the 64 positions is outside [-2^51, 2^51)
 template <int HD>
 __global__ __launch_bounds__(256) void k_pfa_prep(uint8_t *__restrict__ KD,
-                                                 uint8_t *__restrict__ VD,
                                                  uint64_t *__restrict__ CK,
-                                                 uint64_t *__restrict__ VS,
-                                                 uint2 *__restrict__ VL,
+                                                 double *__restrict__ VF,
+                                                 int *__restrict__ VB,
                                                  const int64_t *__restrict__ kcache,
                                                  const int64_t *__restrict__ vcache, int layer,
                                                  int P, int Ppad, int n_kv, int max_seq)
@@ -86,8 +85,6 @@ __global__ __launch_bounds__(256) void k_pfa_prep(uint8_t *__restrict__ KD,
     const int64_t *kb = kcache + (size_t)layer * max_seq * kvd + (size_t)kh * HD;
     const int64_t *vb = vcache + (size_t)layer * max_seq * kvd + (size_t)kh * HD;
     uint8_t *kd = KD + (size_t)kh * 8 * Ppad * HDP;
-    uint8_t *vd = VD + (size_t)kh * 8 * HD * Ppad;
-    uint2 *vl = VL + (size_t)kh * Ppad * HD;
 
     // keys: (position, 4 dims) per item
     for (int it = tid; it < PF_STEP * (HDP / 4); it += 256) {
@@ -102,22 +99,16 @@ __global__ __launch_bounds__(256) void k_pfa_prep(uint8_t *__restrict__ KD,
         for (int a = 0; a < 8; ++a)
             *reinterpret_cast<uint32_t *>(kd + ((size_t)a * Ppad + j) * HDP + d) = w[a];
     }
-    // values: (dim, 4 positions) per item, the dims of a wave consecutive
-    for (int it = tid; it < HD * (PF_STEP / 4); it += 256) {
-        const int d = it % HD, j = j0 + 4 * (it / HD);
-        uint64_t v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            v[e] = j + e < P ? (uint64_t)vb[(size_t)(j + e) * kvd + d] : kDig;
-        uint32_t w[8];
-        digits4(v, w);
-#pragma unroll
-        for (int a = 0; a < 8; ++a)
-            *reinterpret_cast<uint32_t *>(vd + ((size_t)a * HD + d) * Ppad + j) = w[a];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            vl[(size_t)(j + e) * HD + d] = j + e < P ? low_limbs(v[e]) : make_uint2(0, 0);
+    uint32_t big = 0;
+#pragma unroll 4
+    for (int it = tid; it < PF_STEP * HD; it += 256) {
+        const int j = j0 + it / HD, d = it % HD;
+        const int64_t v = j < P ? vb[(size_t)j * kvd + d] : 0;
+        VF[((size_t)kh * Ppad + j) * HD + d] = q48_f51(v, big);
     }
+    const int any = __syncthreads_or(q48_f51_big(big));
+    if (tid == 0)
+        VB[(size_t)kh * (Ppad / PF_STEP) + c] = any ? 1 : 0;
     if (tid < PF_STEP) {
         const int j = j0 + tid;
         q48_u128 s = 0;
@@ -127,12 +118,6 @@ __global__ __launch_bounds__(256) void k_pfa_prep(uint8_t *__restrict__ KD,
             s = s * kDig - (q48_u128)kDig * kDig * (q48_u128)HD;
         }
         st128(CK + 2 * ((size_t)kh * Ppad + j), s);
-    } else if (tid < PF_STEP + HD) {
-        const int d = tid - PF_STEP;
-        q48_u128 s = 0;
-        for (int j = j0; j < j0 + PF_STEP; ++j)
-            s += j < P ? (q48_u128)(q48_i128)vb[(size_t)j * kvd + d] : (q48_u128)kDig;
-        st128(VS + 2 * (((size_t)kh * (Ppad / PF_STEP) + c) * HD + d), s);
     }
 }
 
@@ -143,34 +128,39 @@ __global__ __launch_bounds__(256) void k_pfa_prep(uint8_t *__restrict__ KD,
 //  phase 1: scores by MFMA (wave w: position tiles w, w + 4, ...), written to
 //           the block's workspace rows, and the row maxima;
 //  phase 2: exponentials in place and the row sums;
-//  phase 3: per 64 positions, the weights p (fp_div) as digits and limbs in
-//           LDS, the values' limbs in LDS; X by MFMA (wave w: dims 16 w ..),
-//           Λ on the VALU (wave w: rows 4 w ..);
-//  then o = (X - 2^24 Λ) >> 48.
+//  phase 3: wave w takes the 16-position chunks w, w + 4, ... by itself, with
+//           no barrier: the weights of its 16 rows (fp_div, four a lane) go
+//           through LDS so that lane l of each row of 16 lanes holds position
+//           l % 16 of every query row, and row_newbcast hands them to the
+//           lanes, which hold one dim each (head_dim 128: two; 32: 32
+//           positions a chunk, 16 for each half of the wave) of the chunk's
+//           values and the sums of all 16 rows: 256 FP64 operations a chunk
+//           on 16 value loads and 16 LDS reads;
+//  then the four waves' sums are added in LDS.
+// TinyLlama heads, rows 0..1499: 1028 -> 474 us a launch against digit
+// products of weights and values on the matrix cores with six integer
+// operations per term for the truncations (and two barriers per 64
+// positions); rows 512..1023: 390 -> 205 us.  158 VGPRs (228) and 17 KB of
+// LDS (59) let three blocks run on a compute unit (two).
 template <int HD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 128 ? 1 : 2))) void
-k_pfa(int64_t *__restrict__ out,
-                                            const int64_t *__restrict__ QKV,
-                                            const uint8_t *__restrict__ KD,
-                                            const uint8_t *__restrict__ VD,
-                                            const uint64_t *__restrict__ CK,
-                                            const uint64_t *__restrict__ VS,
-                                            const uint2 *__restrict__ VL,
-                                            int64_t *__restrict__ SCR,
-                                            const int64_t *__restrict__ scale_p, int p0, int T,
-                                            int n_heads, int n_kv, int Ppad, size_t per_head)
+k_pfa(int64_t *__restrict__ out, const int64_t *__restrict__ QKV,
+      const uint8_t *__restrict__ KD, const uint64_t *__restrict__ CK,
+      const double *__restrict__ VF, const int *__restrict__ VB,
+      const int64_t *__restrict__ vcache, int64_t *__restrict__ SCR,
+      const int64_t *__restrict__ scale_p, int p0, int T, int n_heads, int n_kv, int Ppad,
+      size_t per_head)
 {
     q48_round_down();
     constexpr int HDP = HD < 64 ? 64 : HD, KS = HDP / 64;
-    constexpr int NDT = HD / 16, DTW = (NDT + 3) / 4;   // 16-dim tiles, per wave
-    constexpr int DB = HD / 4, JG = 64 / DB, JPER = PF_STEP / JG;
-    static_assert(DB * JG == 64 && HD % 16 == 0, "lane split");
-    __shared__ __align__(16) uint8_t pd[8][PF_ROWS][PF_STEP];   // weight digits of a step
-    __shared__ __align__(16) uint2 pl[PF_ROWS][PF_STEP];        // weight limbs of a step
-    __shared__ __align__(16) uint2 vl[PF_STEP][HD];             // value limbs of a step
-    __shared__ uint64_t lam[PF_ROWS][HD];
-    __shared__ q48_u128 cq[PF_ROWS], cp[PF_ROWS], cv[HD];
+    constexpr int DL = HD == 128 ? 2 : 1;          // dims per lane
+    constexpr int PG = HD == 32 ? 2 : 1;           // 16-position groups per chunk
+    constexpr int CP = 16 * PG;                    // positions per chunk
+    __shared__ double pw[4][PF_ROWS][CP];          // a wave's weights of a chunk
+    __shared__ uint64_t lam[PF_ROWS][HD];          // the sums
+    __shared__ q48_u128 cq[PF_ROWS];
     __shared__ int64_t mxs[4][PF_ROWS], sums[PF_ROWS];
+    __shared__ int form;                           // see phase 3
 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int rl = lane & 15, kq = lane >> 4;
@@ -238,6 +228,10 @@ k_pfa(int64_t *__restrict__ out,
         if (w == 0 && kq == 0)
             cq[rl] = qs * kDig;
     }
+    if (tid == 0)
+        form = 0;
+    for (int i = tid; i < PF_ROWS * HD; i += 256)
+        (&lam[0][0])[i] = 0;
     __syncthreads();
 
     // phase 1: lane holds position j0 + rl of rows 4 kq + i
@@ -292,6 +286,7 @@ k_pfa(int64_t *__restrict__ out,
     {
         const int r = tid >> 4, jj = tid & 15;
         int64_t sum = 0;
+        int odd = 0;   // an exponential outside [0, ONE]: a wrapped difference
         if (r < nrow) {
             int64_t m = mxs[0][r];
 #pragma unroll
@@ -302,6 +297,7 @@ k_pfa(int64_t *__restrict__ out,
             auto ex = [&](int j) {
                 const int64_t e = q48_safe_exp((int64_t)((uint64_t)srow[j] - (uint64_t)m));
                 srow[j] = e;
+                odd |= (uint64_t)e > (uint64_t)Q48_ONE ? 1 : 0;
                 return e;
             };
             int j = jj;
@@ -316,182 +312,168 @@ k_pfa(int64_t *__restrict__ out,
         sum = (int64_t)group_sum64<16>((uint64_t)sum);
         if (jj == 0)
             sums[r] = sum;
+        // a value outside [-2^51, 2^51) somewhere in the span
+        const int *vbig = VB + (size_t)kh * (Ppad / PF_STEP);
+        for (int c = tid; c < J / PF_STEP; c += 256)
+            odd |= vbig[c] ? 2 : 0;
+        if (odd)
+            atomicOr(&form, odd);
     }
     __syncthreads();
 
-    // phase 3: per step of 64 positions the step's weights are in pd / pl and
-    // its value limbs in vl.  Before the low-part loop each thread loads the
-    // next step's exponentials and its wave's value digits of this step; after
-    // the step's barrier the next value limbs go straight to LDS
-    // (global_load_lds) while the next weights are divided.
-    const int r3 = tid >> 4, q4 = tid & 15;
-    const int S3 = p0 + t0 + r3 + 1;
-    const bool rv = r3 < nrow;
-    const int64_t den = sums[r3];
-    const q48_divisor dvr = q48_divisor_of(den);
-    const int db = lane / JG, jg = lane % JG;
-    constexpr int FLUSH = 128 / JPER;   // steps between flushes of the 32-bit Λ sums (< 2^31)
-    const uint8_t *vd = VD + (size_t)kh * 8 * HD * Ppad;
-    const char *vlg = reinterpret_cast<const char *>(VL + (size_t)kh * Ppad * HD);
-    q48_u128 psum = 0;
-    uint64_t er[4] = {0, 0, 0, 0};
-    auto load_e = [&](int j0) {
-        if (rv) {
-            const ulonglong2 *e2 =
-                reinterpret_cast<const ulonglong2 *>(sc + (size_t)r3 * J + j0 + 4 * q4);
-            const ulonglong2 u0 = e2[0], u1 = e2[1];
-            er[0] = u0.x;
-            er[1] = u0.y;
-            er[2] = u1.x;
-            er[3] = u1.y;
-        }
-    };
-    // weights of row r3 at positions j0 + 4 q4 .. + 3 (0 past the row's position)
-    auto weights = [&](int j0) {
-        const int jb = j0 + 4 * q4;
-        uint64_t p[4] = {0, 0, 0, 0};
-        if (rv) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (jb + k < S3)
-                    p[k] = (uint64_t)(den > 0 ? q48_div_by((int64_t)er[k], dvr) : (int64_t)er[k]);
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            psum += p[k];
-        uint32_t wd[8];
-        digits4(p, wd);
-#pragma unroll
-        for (int a = 0; a < 8; ++a)
-            *reinterpret_cast<uint32_t *>(&pd[a][r3][4 * q4]) = wd[a];
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            pl[r3][4 * q4 + k] = low_limbs(p[k]);
-    };
-    // value limbs of positions j0 .. j0 + 63: 512 HD contiguous bytes, 1 KiB
-    // per wave and instruction
-    auto load_vl = [&](int j0) {
-        const char *src = vlg + (size_t)j0 * HD * sizeof(uint2) + 16 * tid;
-        char *dst = reinterpret_cast<char *>(&vl[0][0]) + 1024 * w;
-#pragma unroll
-        for (int i = 0; i < HD / 8; ++i)
-            __builtin_amdgcn_global_load_lds(src + 4096 * i, dst + 4096 * i, 16, 0, 0);
-    };
-    for (int i = tid; i < PF_ROWS * HD; i += 256)
-        (&lam[0][0])[i] = 0;
-    v4i accp[DTW][14];
-#pragma unroll
-    for (int u = 0; u < DTW; ++u)
-#pragma unroll
-        for (int d = 0; d < 14; ++d)
-            accp[u][d] = (v4i){0, 0, 0, 0};
-    uint32_t t32[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int cc = 0; cc < 4; ++cc)
-            t32[i][cc] = 0;
-    load_vl(0);
-    load_e(0);
-    weights(0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    const int ns = J / PF_STEP;
-    for (int st = 0; st < ns; ++st) {
-        const int j0 = PF_STEP * st;
-        if (st + 1 < ns)
-            load_e(j0 + PF_STEP);
-        v4i Bv[DTW][8];
-#pragma unroll
-        for (int u = 0; u < DTW; ++u)
-            if (w + 4 * u < NDT)
-#pragma unroll
-                for (int b = 0; b < 8; ++b)
-                    Bv[u][b] = *reinterpret_cast<const v4i *>(
-                        vd + ((size_t)b * HD + 16 * (w + 4 * u) + rl) * Ppad + j0 + 16 * kq);
-        // Λ: rows 4 w .. 4 w + 3, dims 4 db .. 4 db + 3, positions j0 + jg + JG k
-#pragma unroll 4
-        for (int k = 0; k < JPER; ++k) {
-            const int jl = jg + JG * k;
-            uint2 a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                a[i] = pl[4 * w + i][jl];
-#pragma unroll
-            for (int cc = 0; cc < 4; ++cc)
-                b[cc] = vl[jl][4 * db + cc];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int cc = 0; cc < 4; ++cc)
-                    t32[i][cc] = trunc_low_acc(a[i], b[cc], t32[i][cc]);
-        }
-        if ((st + 1) % FLUSH == 0 || st + 1 == ns) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int cc = 0; cc < 4; ++cc) {
-                    atomicAdd(reinterpret_cast<unsigned long long *>(&lam[4 * w + i][4 * db + cc]),
-                              (unsigned long long)t32[i][cc]);
-                    t32[i][cc] = 0;
-                }
-        }
-        // X: the wave's 16-dim tiles
-#pragma unroll
-        for (int u = 0; u < DTW; ++u) {
-            if (w + 4 * u < NDT) {
-                v4i Ap[8];
-#pragma unroll
-                for (int a = 0; a < 8; ++a)
-                    Ap[a] = *reinterpret_cast<const v4i *>(&pd[a][rl][16 * kq]);
-#pragma unroll
-                for (int a = 0; a < 8; ++a)
-#pragma unroll
-                    for (int b = 0; b < 8; ++b)
-                        if (a + b <= 13)
-                            accp[u][a + b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-                                Ap[a], Bv[u][b], accp[u][a + b], 0, 0, 0);
+    // phase 3.  form 0: every exponential is in [0, ONE], so each row's sum is
+    // exact, at least ONE, and its weights add up to at most ONE; every value
+    // of the span is in [-2^51, 2^51).  2: the same weights, larger values.
+    // Bit 0: weights of any kind.
+    const int vform = form;
+    const int Smax = p0 + t0 + nrow;
+    const size_t kvd = (size_t)n_kv * HD;
+    const int64_t *vraw = vcache + (size_t)kh * HD;
+    if (vform & 1) {
+        // the weights in place of the exponentials, then integer products
+        {
+            const int r = tid >> 4;
+            if (r < nrow) {
+                const int64_t den = sums[r];
+                const q48_divisor dv = q48_divisor_of(den);
+                if (den > 0)
+                    for (int j = tid & 15; j < p0 + t0 + r + 1; j += 16)
+                        sc[(size_t)r * J + j] = q48_div_by(sc[(size_t)r * J + j], dv);
             }
         }
         __syncthreads();
-        if (st + 1 < ns) {
-            load_vl(j0 + PF_STEP);
-            weights(j0 + PF_STEP);
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
+        for (int i = tid; i < nrow * HD; i += 256) {
+            const int r = i / HD, d = i % HD;
+            uint64_t a = 0;
+            for (int j = 0; j < p0 + t0 + r + 1; ++j)
+                a += (uint64_t)q48_mul(sc[(size_t)r * J + j], vraw[(size_t)j * kvd + d]);
+            lam[r][d] = a;
         }
-    }
-
-    psum = q48_dpp128<Q48_DPP_XOR1>(psum) + psum;
-    psum = q48_dpp128<Q48_DPP_XOR2>(psum) + psum;
-    psum = q48_dpp128<Q48_DPP_HALF_MIRROR>(psum) + psum;
-    psum = q48_dpp128<Q48_DPP_MIRROR>(psum) + psum;
-    if (q4 == 0)
-        cp[r3] = psum * kDig;
-    if (tid < HD) {
-        const uint64_t *vs = VS + 2 * ((size_t)kh * (Ppad / PF_STEP) * HD + tid);
-        q48_u128 s = 0;
-        for (int c = 0; c < J / PF_STEP; ++c)
-            s += ld128(vs + 2 * (size_t)c * HD);
-        cv[tid] = s * kDig - (q48_u128)kDig * kDig * (q48_u128)(uint64_t)J;
+    } else {
+        const int g = lane >> 4;
+        double y48[4];
+        uint64_t den[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const q48_divisor dv = q48_divisor_of(4 * i + g < nrow ? sums[4 * i + g] : Q48_ONE);
+            y48[i] = dv.y48;
+            den[i] = dv.d;
+        }
+        const double *vf = VF + (size_t)kh * Ppad * HD;
+        const int vd = HD == 32 ? lane & 31 : lane;         // this lane's dim (and + 64)
+        const int vp = HD == 32 ? 16 * (lane >> 5) : 0;     // its positions in the chunk
+        // one set of sums over the span: the weights and values as this pass
+        // takes them (0: p 2^-48 and v; 1: p 2^-48 and v mod 2^48; 2, 3: the
+        // low 24 bits and the rest of p, and v >> 48), shifted left by sh
+        auto pass = [&](auto split, int mode) {
+            constexpr bool SPLIT = decltype(split)::value;
+            double acc[DL][PF_ROWS];
+#pragma unroll
+            for (int l = 0; l < DL; ++l)
+#pragma unroll
+                for (int r = 0; r < PF_ROWS; ++r)
+                    acc[l][r] = Q48_FSUM0;
+            uint64_t er[4 * PG];
+            auto load_e = [&](int j0) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int u = 0; u < PG; ++u)
+                        er[PG * i + u] =
+                            (uint64_t)sc[(size_t)(4 * i + g) * J + j0 + 16 * u + rl];
+            };
+            if (CP * w < Smax)
+                load_e(CP * w);
+            for (int j0 = CP * w; j0 < Smax; j0 += 4 * CP) {
+                double v[DL][16];
+#pragma unroll
+                for (int n = 0; n < 16; ++n)
+#pragma unroll
+                    for (int l = 0; l < DL; ++l) {
+                        const int j = j0 + vp + n;
+                        if constexpr (SPLIT) {
+                            const int64_t x = vraw[(size_t)min(j, Smax - 1) * kvd + vd + 64 * l];
+                            uint32_t any = 0;
+                            v[l][n] = q48_f51(mode == 1 ? x & (Q48_ONE - 1) : x >> 48, any);
+                        } else {
+                            v[l][n] = vf[(size_t)j * HD + vd + 64 * l];
+                        }
+                    }
+                // fp_div(e, sum), as q48_div_by (0 <= e <= ONE <= sum, so its
+                // estimate settles), as p 2^-48; 0 past the row's position
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int u = 0; u < PG; ++u) {
+                        const uint64_t e = er[PG * i + u];
+                        const int j = j0 + 16 * u + rl, r = 4 * i + g;
+                        const double ed =
+                            __builtin_bit_cast(double, e | 0x4330000000000000ull) - 0x1p52;
+                        const uint64_t q0 =
+                            q48_word_m52(__builtin_fma(ed, y48[i], 0x1p52 - 0.5));
+                        const uint64_t rem = (e << 48) - q0 * den[i];
+                        const double p = q48_pscaled((int64_t)(q0 + (rem >= den[i] ? 1 : 0)));
+                        pw[w][r][16 * u + rl] = r < nrow && j < p0 + t0 + r + 1 ? p : 0.0;
+                    }
+                if (j0 + 4 * CP < Smax)
+                    load_e(j0 + 4 * CP);
+                // the wave's own LDS writes before its reads (in order; the
+                // fence keeps the compiler's order)
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+                for (int r = 0; r < PF_ROWS; r += 4) {
+                    double p[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        p[i] = pw[w][r + i][vp + rl];
+                        if constexpr (SPLIT)
+                            if (mode >= 2) {
+                                const double pb = __builtin_fma(p[i], 0x1p24, 0x1p52) - 0x1p52;
+                                p[i] = mode == 3 ? pb
+                                                 : __builtin_fma(p[i], 0x1p48, -pb * 0x1p24);
+                            }
+                    }
+#pragma unroll
+                    for (int l = 0; l < DL; ++l) {
+                        auto f4 = [&](auto base) {
+                            constexpr int B = decltype(base)::value;
+                            const double x[4] = {v[l][B], v[l][B + 1], v[l][B + 2], v[l][B + 3]};
+                            q48_fsum4x4<B>(acc[l][r], acc[l][r + 1], acc[l][r + 2], acc[l][r + 3],
+                                           p, x);
+                        };
+                        f4(std::integral_constant<int, 0>{});
+                        f4(std::integral_constant<int, 4>{});
+                        f4(std::integral_constant<int, 8>{});
+                        f4(std::integral_constant<int, 12>{});
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            }
+#pragma unroll
+            for (int r = 0; r < PF_ROWS; ++r)
+#pragma unroll
+                for (int l = 0; l < DL; ++l) {
+                    uint64_t t = (uint64_t)q48_fsum_total(acc[l][r]);
+                    if (SPLIT && mode == 3)
+                        t <<= 24;
+                    atomicAdd(reinterpret_cast<unsigned long long *>(&lam[r][vd + 64 * l]),
+                              (unsigned long long)t);
+                }
+        };
+        if (vform == 0)
+            pass(std::false_type{}, 0);
+        else
+            for (int mode = 1; mode <= 3; ++mode)
+                pass(std::true_type{}, mode);
     }
     __syncthreads();
-#pragma unroll
-    for (int u = 0; u < DTW; ++u) {
-        const int dt = w + 4 * u;
-        if (dt < NDT) {
-            const int d = 16 * dt + rl;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = 4 * kq + i;
-                if (m < nrow) {
-                    const q48_u128 X = digits_total(accp[u], i) + cp[m] + cv[d];
-                    const q48_u128 o = X - ((q48_u128)lam[m][d] << 24);
-                    out[(size_t)(t0 + m) * n_heads * HD + (size_t)h * HD + d] = (int64_t)(o >> 48);
-                }
-            }
-        }
-    }
+    for (int i = tid; i < nrow * HD; i += 256)
+        out[(size_t)(t0 + i / HD) * n_heads * HD + (size_t)h * HD + i % HD] =
+            (int64_t)lam[i / HD][i % HD];
 }
 
 } // namespace
@@ -520,19 +502,20 @@ int q48_launch_pf_attn_mfma(q48_ctx *c, int64_t *out, const int64_t *QKV, int64_
         return at;
     };
     const size_t o_kd = take((size_t)n_kv * 8 * Ppad * HDP);
-    const size_t o_vd = take((size_t)n_kv * 8 * hd * Ppad);
     const size_t o_ck = take((size_t)n_kv * Ppad * 16);
-    const size_t o_vs = take((size_t)n_kv * (Ppad / PF_STEP) * hd * 16);
-    const size_t o_vl = take((size_t)n_kv * Ppad * hd * sizeof(uint2));
+    const size_t o_vf = take((size_t)n_kv * Ppad * hd * sizeof(double));
+    const size_t o_vb = take((size_t)n_kv * (Ppad / PF_STEP) * sizeof(int));
     const size_t o_sc = take((size_t)n_heads * per_head * sizeof(int64_t));
     int rc = q48_ws_reserve(c, o);
     if (rc)
         return rc;
     uint8_t *ws = (uint8_t *)c->ws;
-    uint8_t *KD = ws + o_kd, *VD = ws + o_vd;
-    uint64_t *CK = (uint64_t *)(ws + o_ck), *VS = (uint64_t *)(ws + o_vs);
-    uint2 *VL = (uint2 *)(ws + o_vl);
+    uint8_t *KD = ws + o_kd;
+    uint64_t *CK = (uint64_t *)(ws + o_ck);
+    double *VF = (double *)(ws + o_vf);
+    int *VB = (int *)(ws + o_vb);
     int64_t *SCR = (int64_t *)(ws + o_sc);
+    const int64_t *vl = vcache + (size_t)layer * max_seq * n_kv * hd;
     const int64_t *scale_p = c->rope_sin + (size_t)c->rope_max_seq * (c->rope_head_dim / 2);
     const dim3 pgrid(Ppad / PF_STEP, n_kv);
     const unsigned grid = 8 % n_kv == 0
@@ -540,10 +523,10 @@ int q48_launch_pf_attn_mfma(q48_ctx *c, int64_t *out, const int64_t *QKV, int64_
                               : (unsigned)(n_heads * nt);
 #define PFA_LAUNCH(HDV)                                                                       \
     do {                                                                                      \
-        hipLaunchKernelGGL(k_pfa_prep<HDV>, pgrid, dim3(256), 0, c->stream, KD, VD, CK, VS,   \
-                           VL, kcache, vcache, layer, P, Ppad, n_kv, max_seq);                \
-        hipLaunchKernelGGL(k_pfa<HDV>, dim3(grid), dim3(256), 0, c->stream, out, QKV, KD, VD, \
-                           CK, VS, VL, SCR, scale_p, p0, T, n_heads, n_kv, Ppad, per_head);   \
+        hipLaunchKernelGGL(k_pfa_prep<HDV>, pgrid, dim3(256), 0, c->stream, KD, CK, VF, VB,   \
+                           kcache, vcache, layer, P, Ppad, n_kv, max_seq);                    \
+        hipLaunchKernelGGL(k_pfa<HDV>, dim3(grid), dim3(256), 0, c->stream, out, QKV, KD, CK, \
+                           VF, VB, vl, SCR, scale_p, p0, T, n_heads, n_kv, Ppad, per_head);   \
     } while (0)
     if (hd == 64)
         PFA_LAUNCH(64);
