@@ -275,14 +275,26 @@ __device__ __forceinline__ void mfma_plane8(v16i (&acc)[14], const uint8_t *xs,
 // to give every XCD a contiguous range, and that range is walked in groups of
 // GROUP row tiles: a group's W tiles stay in cache while its token tiles pass.
 constexpr int GROUP = 8;
-__device__ __forceinline__ void tile_of(int b, int nn, int nt, int &n_tile, int &t_tile)
+__host__ __device__ __forceinline__ void tile_of(int b, int nn, int nt, int &n_tile, int &t_tile)
 {
     const int total = nn * nt, q = total / 8, r = total % 8, x = b % 8, l = b / 8;
     const int pid = x < r ? x * (q + 1) + l : r * (q + 1) + (x - r) * q + l;
     const int per = GROUP * nt, g = pid / per, first = g * GROUP;
-    const int gs = min(nn - first, GROUP), in = pid - g * per;
+    const int gs = nn - first < GROUP ? nn - first : GROUP, in = pid - g * per;
     n_tile = first + in % gs;
     t_tile = in / gs;
+}
+
+// The block whose tile is (n_tile, t_tile): tile_of's inverse.
+__host__ __device__ inline int block_of(int n_tile, int t_tile, int nn, int nt)
+{
+    const int total = nn * nt, q = total / 8, r = total % 8;
+    const int g = n_tile / GROUP, first = g * GROUP;
+    const int gs = nn - first < GROUP ? nn - first : GROUP;
+    const int pid = first * nt + t_tile * gs + (n_tile - first);
+    const int x = pid < r * (q + 1) ? pid / (q + 1) : r + (pid - r * (q + 1)) / (q > 0 ? q : 1);
+    const int l = pid < r * (q + 1) ? pid % (q + 1) : (pid - r * (q + 1)) % (q > 0 ? q : 1);
+    return 8 * l + x;
 }
 
 // Register i of the 14 digit-sum accumulators as the 128-bit sum
@@ -650,6 +662,61 @@ __global__ __launch_bounds__(256) void k_gemm_i8_reduce(int64_t *__restrict__ Y,
 // into LDS by DMA (global_load_lds), so the k loop runs no digit split.
 // ---------------------------------------------------------------------------
 
+// The shift of each 64-row tile's planes (k_planes) from its largest
+// magnitude, left in bits 16..18 of the row tile's first mask word: one block
+// per row tile.
+__global__ __launch_bounds__(1024) void k_tile_shift(uint32_t *__restrict__ mask,
+                                                    const int64_t *__restrict__ src, int R,
+                                                    int K, int nsteps)
+{
+    __shared__ uint64_t red[16];
+    const int tid = threadIdx.x, r0 = (int)blockIdx.x * MN, r1 = min(r0 + MN, R);
+    const int64_t *p = src + (size_t)r0 * K;
+    const size_t n = (size_t)(r1 - r0) * K;
+    uint64_t mx = 0;
+    auto add = [&](uint64_t v) {
+        const uint64_t a = (int64_t)v < 0 ? (uint64_t)0 - v : v;
+        mx = a > mx ? a : mx;
+    };
+    size_t i0 = 0;
+    if ((((uintptr_t)p) & 15) == 0) {
+        const ulonglong2 *q = reinterpret_cast<const ulonglong2 *>(p);
+        const size_t n4 = n / 8192;   // groups of four 16-byte loads a thread
+        for (size_t g = 0; g < n4; ++g) {
+            ulonglong2 u[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                u[e] = q[4096 * g + 1024 * e + tid];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                add(u[e].x);
+                add(u[e].y);
+            }
+        }
+        i0 = 8192 * n4;
+    }
+    for (size_t i = i0 + tid; i < n; i += 1024)
+        add((uint64_t)p[i]);
+    mx = (uint64_t)q48_wave_max64((int64_t)(mx >> 1));   // halved: 2^63 stays positive
+    if ((tid & 63) == 0)
+        red[tid >> 6] = mx;
+    __syncthreads();
+    if (tid == 0) {
+        for (int i = 1; i < 16; ++i)
+            mx = red[i] > mx ? red[i] : mx;
+        mx = 2 * mx + 1;   // at least the largest magnitude
+        // the lowest plane h <= 6 whose digits reach mx (values up to
+        // sum_{i<=h} 127 256^i), and the largest shift that stays within it
+        uint64_t lim = 127;
+        for (int h = 0; h < 6 && mx > lim; ++h)
+            lim = lim * 256 + 127;
+        uint32_t sh = 0;
+        while (sh < 7 && (mx << (sh + 1)) <= lim)
+            ++sh;
+        mask[(size_t)blockIdx.x * nsteps] = mx <= lim ? sh << 16 : 0;
+    }
+}
+
 // Digit planes of a row-major int64 matrix (R rows, K columns) in the LDS
 // stage order of the window kernels: per row tile rt (64 rows) and k-step s
 // (32 columns), block rt * nsteps + s holds planes 0..7 of the nine-digit
@@ -657,16 +724,29 @@ __global__ __launch_bounds__(256) void k_gemm_i8_reduce(int64_t *__restrict__ Y,
 // past R and columns past K are zero), and mask[rt * nsteps + s] has bit a
 // when plane a holds a nonzero digit and bit 8 when a value may have
 // overflowed v + C (high word >= 0x7F7F7F7F; plane 8 itself is not stored).
-__global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst,
-                                               uint32_t *__restrict__ mask,
+// pitch: blocks per row tile, one past nsteps holding zero planes (X: nsteps + 1,
+// for the steps that fill up the k loop's groups of four; W: nsteps).
+// shifted: the row tile's values are multiplied by 2^shift before the split
+// (bits 16..18 of its first mask word, from k_tile_shift; every mask of the
+// row tile keeps them, so a block may read them before or after the first
+// block writes its own mask), so that the largest one fills its top plane: a
+// bfloat16 weight's low bits then reach down to fewer planes (N(0, 0.02)
+// weights: 10% of the 64 x 32 tiles need a fourth plane, 34% unshifted).
+__global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst, uint32_t *mask,
                                                const int64_t *__restrict__ src, int R, int K,
-                                               int nsteps)
+                                               int nsteps, int pitch, int shifted)
 {
     __shared__ uint32_t red[4];
     const int tid = threadIdx.x;
-    const int rt = (int)blockIdx.x / nsteps, st = (int)blockIdx.x % nsteps;
+    const int rt = (int)blockIdx.x / pitch, st = (int)blockIdx.x % pitch;
     const Piece pc = piece(tid);
     const int row = rt * MN + pc.r, k0 = st * MK + pc.k8;
+    if (st >= nsteps) {   // padding: zero planes, no mask
+        for (int i = tid; i < PLANE / 2; i += 256)
+            reinterpret_cast<uint4 *>(dst + (size_t)blockIdx.x * 8 * PLANE)[i] =
+                make_uint4(0, 0, 0, 0);
+        return;
+    }
     uint64_t v[8];
     const int64_t *rp = src + (size_t)min(row, R - 1) * K + k0;
     if (row < R && k0 + 8 <= K && (((uintptr_t)rp) & 15) == 0) {
@@ -682,6 +762,14 @@ __global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst,
         for (int e = 0; e < 8; ++e)
             v[e] = row < R && k0 + e < K ? (uint64_t)rp[e] : 0;
     }
+    const uint32_t sh =
+        shifted ? (__hip_atomic_load(mask + (size_t)rt * nsteps, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT) >> 16) & 7u
+                : 0u;
+    if (sh)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            v[e] <<= sh;
     uint64_t u[8];
     bool big = false;
 #pragma unroll
@@ -705,7 +793,7 @@ __global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst,
         d[4 + a] = make_uint2(h0[a] ^ 0x80808080u, h1[a] ^ 0x80808080u);
     d[7] = make_uint2(h0[3], h1[3]);
     uint8_t *p = dst + (size_t)blockIdx.x * 8 * PLANE + pc.off;
-    uint32_t m = big ? 0x100u : 0u;
+    uint32_t m = (big ? 0x100u : 0u) | (sh << 16);
 #pragma unroll
     for (int a = 0; a < 8; ++a) {
         *reinterpret_cast<uint2 *>(p + a * PLANE) = d[a];
@@ -716,11 +804,15 @@ __global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst,
         red[tid >> 6] = m;
     __syncthreads();
     if (tid == 0)
-        mask[blockIdx.x] = red[0] | red[1] | red[2] | red[3];
+        mask[(size_t)rt * nsteps + st] = red[0] | red[1] | red[2] | red[3];
 }
 
-// One LDS stage of the planes path: X planes 0..6, then W planes WP0 .. WP0 + 4.
-constexpr int PX_BYTES = 7 * PLANE, PSTAGE = 12 * PLANE;
+// One LDS stage of the planes path, NW row tiles of W: X planes 0..6, then W
+// planes TOP - 2 .. TOP of each row tile, then plane TOP - 3 of each; whole slots
+// of four 1 KB chunks, one per wave.
+constexpr int PX_BYTES = 7 * PLANE;
+constexpr int stage_slots(int nw) { return (14 + 8 * nw + 3) / 4; }
+constexpr int stage_bytes(int nw) { return 4096 * stage_slots(nw); }
 
 // s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding)
 template <int N>
@@ -729,8 +821,6 @@ __device__ __forceinline__ void wait_vm()
     static_assert(N >= 0 && N < 64, "vmcnt");
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
-
-typedef const __attribute__((address_space(4))) uint32_t *ConstMask;
 
 // Workgroup barrier without the fence of __syncthreads (whose release waits
 // for every DMA still in flight); the caller's s_waitcnt before it decides
@@ -743,183 +833,388 @@ __device__ __forceinline__ void stage_barrier()
     asm volatile("" ::: "memory");
 }
 
-// The k loop of one window (LO) over a ring of four LDS stages.  Step i:
+// The k loop over a ring of four LDS stages.  Step i:
 //   wait for step i + 1's DMA (this wave's), barrier (every wave's);
-//   DMA step i + 3 into the stage step i - 1 used (each wave moves six 1 KB
+//   DMA step i + 3 into the stage step i - 1 used (each wave moves CPW 1 KB
 //   chunks: 64 lanes x 16 bytes);
-//   read step i + 1's operands into the spare register set, while the MFMAs
-//   of step i run on the set read during step i - 1.
+//   run the MFMAs of step i on the operands read during step i - 1, while
+//   reading step i + 1's.
 // The stages are four LDS objects named statically in each step (the loop
 // is unrolled by four), so the compiler's own waits for the reads of one
 // stage do not count the DMA into another.
-template <int LO>
-__device__ __forceinline__ void planes_pass(uint8_t (&s0)[PSTAGE], uint8_t (&s1)[PSTAGE],
-                                            uint8_t (&s2)[PSTAGE], uint8_t (&s3)[PSTAGE],
-                                            ConstMask wm, const uint8_t *xsrc,
-                                            const uint8_t *wsrc, int ns, bool rev,
-                                            v16i (&acc)[14])
+//
+// wsrc points at plane TOP - 4 of each row tile, and digit sums are kept
+// relative to it: acc[j][r] is the sum of weight 256^(TOP - 4 + r), so one code
+// serves every window.  A step multiplies X planes 0..6 by W planes TOP - 2
+// .. TOP, 21 NW MFMAs, and by plane TOP - 3 only for a row tile that holds a
+// digit there (7 more; the shift of k_planes makes that about one step in ten
+// for bfloat16 weights).  ext (LDS) tells, a byte for each loop step, zero past
+// the last: bit n row tile n's plane TOP - 3, bit 2 some plane TOP - 4.  The
+// chunks of plane TOP - 3 are moved only then: otherwise their slots re-read a
+// fixed line set that stays in the vector cache, so that every step issues the
+// same number of DMAs with no branch around one, which would make the compiler
+// wait for all of them.  Plane TOP - 4 (one step in thousands) is loaded where
+// it is needed.
+// acc[n][r] += A B.  The digit sums of two row tiles take 352 registers, more
+// than the 256 accumulation registers the compiler keeps MFMA results in, so
+// with NW = 2 the instruction is written out with the register file chosen per
+// sum: the first row tile's and sums 0..3 of the second in accumulation
+// registers, the rest in vector registers.  s_nop 1: the wait states a vector
+// write of an operand needs before an MFMA reads it (the compiler inserts
+// them only for instructions it knows).
+template <bool AG>
+__device__ __forceinline__ void mfma_asm(v16i &c, const v4i &a, const v4i &b)
 {
-    constexpr int WP0 = LO > 0 ? LO - 1 : 0;   // first W plane in the stage
-    constexpr int NB = LO > 0 ? 5 : 4;         // W planes the MFMAs read
+    if constexpr (AG)
+        asm("s_nop 1\n\tv_mfma_i32_32x32x32_i8 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    else
+        asm("s_nop 1\n\tv_mfma_i32_32x32x32_i8 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+template <int NW>
+__device__ __forceinline__ void mfma_i8(v16i (&acc)[NW][11], int n, int r, const v4i &a,
+                                        const v4i &b)
+{
+    if constexpr (NW == 1)
+        acc[n][r] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, acc[n][r], 0, 0, 0);
+    else if (n == 0 || r < 4)   // constants once unrolled
+        mfma_asm<true>(acc[n][r], a, b);
+    else
+        mfma_asm<false>(acc[n][r], a, b);
+}
+// The sums after mfma_asm: an MFMA's result may be read by other vector
+// instructions only after its passes (at most 18 wait states), which the
+// compiler does not know of here; what reads a sum depends on this.
+template <int NW>
+__device__ __forceinline__ void mfma_settle(v16i (&acc)[NW][11])
+{
+    if constexpr (NW > 1) {
+        asm volatile("s_nop 15\n\ts_nop 15"
+                     : "+a"(acc[0][0]), "+a"(acc[0][1]), "+a"(acc[0][2]), "+a"(acc[0][3]),
+                       "+a"(acc[0][4]), "+a"(acc[0][5]), "+a"(acc[0][6]), "+a"(acc[0][7]),
+                       "+a"(acc[0][8]), "+a"(acc[0][9]), "+a"(acc[0][10]));
+        asm volatile(""
+                     : "+a"(acc[1][0]), "+a"(acc[1][1]), "+a"(acc[1][2]), "+a"(acc[1][3]),
+                       "+v"(acc[1][4]), "+v"(acc[1][5]), "+v"(acc[1][6]), "+v"(acc[1][7]),
+                       "+v"(acc[1][8]), "+v"(acc[1][9]), "+v"(acc[1][10]));
+    }
+}
+
+// The X chunks of slots 0 .. XSLOTS - 1 (which hold no W) of the loop's steps
+// 0..2, before the masks are known.
+constexpr int XSLOTS = 3;   // chunks 0 .. 11 of 14
+template <int PS>
+__device__ __forceinline__ void planes_first_x(uint8_t (&s0)[PS], uint8_t (&s1)[PS],
+                                               uint8_t (&s2)[PS], const uint8_t *xsrc, int ns,
+                                               int xz, bool rev)
+{
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    auto one = [&](int s, uint8_t(&dst)[PS]) {
+        const uint32_t at = (uint32_t)(s < ns ? (rev ? ns - 1 - s : s) : xz) * (8u * PLANE);
+#pragma unroll
+        for (int j = 0; j < XSLOTS; ++j) {
+            const int c = w + 4 * j;
+            __builtin_amdgcn_global_load_lds(xsrc + c * 1024 + (at + (uint32_t)lane * 16u),
+                                             dst + c * 1024, 16, 0, 0);
+        }
+    };
+    one(0, s0);
+    one(1, s1);
+    one(2, s2);
+}
+
+template <int NW>
+__device__ __forceinline__ void planes_pass(uint8_t (&s0)[stage_bytes(NW)],
+                                            uint8_t (&s1)[stage_bytes(NW)],
+                                            uint8_t (&s2)[stage_bytes(NW)],
+                                            uint8_t (&s3)[stage_bytes(NW)],
+                                            const uint8_t *ext, const uint8_t *xsrc,
+                                            const uint8_t *const (&wsrc)[NW], int ns, int xz,
+                                            bool rev, v16i (&acc)[NW][11])
+{
+    constexpr int PSTAGE = stage_bytes(NW);
+    constexpr int DENSE = 14 + 6 * NW;                 // chunks every step moves
+    constexpr int ALL = DENSE + 2 * NW;                // and the conditional ones
+    constexpr int CPW = stage_slots(NW);
+    constexpr int XB = PX_BYTES + 3 * NW * PLANE;      // plane TOP - 3
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wt = w >> 1, wn = w & 1;
     const int off = opnd_off(lane);
-    const uint8_t *ws_src = wsrc + WP0 * PLANE;
-    // step s of the loop is k-step rev ? ns - 1 - s : s of the block's range
-    auto dma = [&](int s, uint8_t(&dst)[PSTAGE]) {
-        s = rev ? ns - 1 - s : s;
+    // this wave's slot j moves chunk w + 4 j: its source in the first k-step (a
+    // scalar address; the k-step's offset is one vector addition a step), and
+    // the ext bit it needs (0: none; 8: past the last chunk)
+    const uint8_t *base[CPW];
+    uint32_t need[CPW];
 #pragma unroll
-        for (int j = 0; j < 6; ++j) {
-            const int c = w + 4 * j;   // chunk 0..23: X 0..13, W 14..23
-            const uint8_t *g = c < 14 ? xsrc + (size_t)s * 8 * PLANE + c * 1024
-                                      : ws_src + (size_t)s * 8 * PLANE + (c - 14) * 1024;
-            __builtin_amdgcn_global_load_lds(g + lane * 16, dst + c * 1024, 16, 0, 0);
-        }
-    };
-    v4i A0[7], B0[NB], A1[7], B1[NB];
-    auto rd = [&](const uint8_t(&src)[PSTAGE], v4i (&A)[7], v4i (&B)[NB]) {
-#pragma unroll
-        for (int a = 0; a < 7; ++a)
-            A[a] = *reinterpret_cast<const v4i *>(src + wt * SLICE + a * PLANE + off);
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-            B[j] = *reinterpret_cast<const v4i *>(src + PX_BYTES + j * PLANE + wn * SLICE + off);
-    };
-    // the step's MFMAs; ext: its W tile reaches plane LO - 1.  The reads of
-    // the next step's operands (issued just before) go out one per MFMA
-    // from the start, so they finish under the MFMAs.
-    auto mult = [&](bool ext, const v4i (&A)[7], const v4i (&B)[NB]) {
-#pragma unroll
-        for (int a = 0; a < 7; ++a)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                acc[a + LO + j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[a], B[LO - WP0 + j],
-                                                                        acc[a + LO + j], 0, 0, 0);
-#pragma unroll
-        for (int k = 0; k < 7 + NB; ++k) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one MFMA
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // one LDS read
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, 28 - 7 - NB, 0);
-        if (LO > 0 && ext) {
-#pragma unroll
-            for (int a = 0; a < 7; ++a)
-                acc[a + WP0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[a], B[0], acc[a + WP0], 0,
-                                                                     0, 0);
-        }
-    };
-    auto ext_of = [&](int i) {
-        uint32_t e = LO > 0 ? wm[rev ? ns - 1 - i : i] : 0;
-        asm volatile("" : "+s"(e));
-        return ((e >> WP0) & 1u) != 0;
-    };
-    // wait until at most n of this wave's chunk DMAs are in flight
-    auto wait_n = [&](int n) {
-        if (n >= 12)
-            wait_vm<12>();
-        else if (n >= 6)
-            wait_vm<6>();
-        else
-            wait_vm<0>();
-    };
-    // prologue: steps 0..2 in flight, step 0 landed and read
-    if (ns > 0)
-        dma(0, s0);
-    if (ns > 1)
-        dma(1, s1);
-    if (ns > 2)
-        dma(2, s2);
-    wait_n(6 * (min(ns, 3) - 1));
-    stage_barrier();
-    if (ns > 0)
-        rd(s0, A0, B0);
-    // steady state: every step has a step i + 3 to load.  The group's four
-    // step masks come in one scalar load at its top, held there by the
-    // empty asm (the wave waits for its operand reads at that point anyway;
-    // a wait in mid-step would also wait for the reads just issued).
-    int i = 0;
-    for (; i + 6 < ns; i += 4) {
-        uint32_t e0 = 0, e1 = 0, e2 = 0, e3 = 0;
-        if (LO > 0) {
-            const ConstMask g = wm + (rev ? ns - 4 - i : i);   // steps i .. i + 3
-            const uint32_t g0 = g[0], g1 = g[1], g2 = g[2], g3 = g[3];
-            e0 = rev ? g3 : g0;
-            e1 = rev ? g2 : g1;
-            e2 = rev ? g1 : g2;
-            e3 = rev ? g0 : g3;
-            asm volatile("" : "+s"(e0), "+s"(e1), "+s"(e2), "+s"(e3));
-        }
-        wait_vm<6>();
-        stage_barrier();
-        dma(i + 3, s3);
-        rd(s1, A1, B1);
-        mult((e0 >> WP0) & 1u, A0, B0);
-        wait_vm<6>();
-        stage_barrier();
-        dma(i + 4, s0);
-        rd(s2, A0, B0);
-        mult((e1 >> WP0) & 1u, A1, B1);
-        wait_vm<6>();
-        stage_barrier();
-        dma(i + 5, s1);
-        rd(s3, A1, B1);
-        mult((e2 >> WP0) & 1u, A0, B0);
-        wait_vm<6>();
-        stage_barrier();
-        dma(i + 6, s2);
-        rd(s0, A0, B0);
-        mult((e3 >> WP0) & 1u, A1, B1);
+    for (int j = 0; j < CPW; ++j) {
+        const int c = w + 4 * j, d = c - 14, x = c - DENSE;
+        const uint8_t *wd = NW > 1 && d >= 6 ? wsrc[NW - 1] : wsrc[0];
+        const uint8_t *wx = NW > 1 && x >= 2 ? wsrc[NW - 1] : wsrc[0];
+        need[j] = c < DENSE ? 0u : c < ALL ? 1u << (x >> 1) : 8u;
+        base[j] = c < 14 ? xsrc + c * 1024
+                  : c < DENSE ? wd + 2 * PLANE + (NW > 1 && d >= 6 ? d - 6 : d) * 1024
+                  : c < ALL ? wx + PLANE + (x & 1) * 1024 : xsrc;
     }
-    // the last zero to six steps (i is a multiple of four: stages continue
-    // the ring)
-    auto tail = [&](int k, uint8_t(&nxt_st)[PSTAGE], uint8_t(&ld_st)[PSTAGE], v4i(&Ac)[7],
-                    v4i(&Bc)[NB], v4i(&An)[7], v4i(&Bn)[NB]) {
-        if (k >= ns)
-            return;
-        wait_n(k + 1 < ns ? 6 * (min(ns - 1, k + 2) - (k + 1)) : 0);
-        stage_barrier();
-        if (k + 3 < ns)
-            dma(k + 3, ld_st);
-        const bool ext = ext_of(k);
-        if (k + 1 < ns)
-            rd(nxt_st, An, Bn);
-        mult(ext, Ac, Bc);
+    // Step s of the loop is k-step rev ? ns - 1 - s : s of the block's range.
+    // The loop runs whole groups of four: steps past the last take the zero X
+    // planes that follow the row tile's (k-step xz), with the last k-step of W.
+    // A conditional slot that is not needed moves its own first k-step.
+    struct Src {
+        uint32_t x, w;   // byte offsets of a step's X and W planes
     };
-    tail(i, s1, s3, A0, B0, A1, B1);
-    tail(i + 1, s2, s0, A1, B1, A0, B0);
-    tail(i + 2, s3, s1, A0, B0, A1, B1);
-    tail(i + 3, s0, s2, A1, B1, A0, B0);
-    tail(i + 4, s1, s3, A0, B0, A1, B1);
-    tail(i + 5, s2, s0, A1, B1, A0, B0);
+    auto src_of = [&](int s) {
+        const int c = min(s, ns - 1), k = rev ? ns - 1 - c : c;
+        return Src{(uint32_t)(s < ns ? k : xz) * (8u * PLANE), (uint32_t)k * (8u * PLANE)};
+    };
+    const uint32_t lane16 = (uint32_t)lane * 16u;
+    auto dma1 = [&](int j, Src f, uint32_t e, uint8_t(&dst)[PSTAGE]) {
+        const int c = w + 4 * j;
+        uint32_t at = 4 * j + 3 < 14 ? f.x : 4 * j >= 14 ? f.w : c < 14 ? f.x : f.w;
+        if (4 * j + 3 >= DENSE)
+            at = need[j] == 0 || (need[j] & e) != 0 ? at : 0u;
+        __builtin_amdgcn_global_load_lds(base[j] + (at + lane16), dst + c * 1024, 16, 0, 0);
+    };
+    auto dma = [&](int s, uint32_t e, uint8_t(&dst)[PSTAGE]) {   // all but the first X slots
+#pragma unroll
+        for (int j = XSLOTS; j < CPW; ++j)
+            dma1(j, src_of(s), e, dst);
+    };
+    // The operands of a step: X planes (A), and the dense W planes and TOP - 3
+    // of each row tile (B).  They are read one step ahead, one LDS read per
+    // MFMA or two from the step's start, so the reads finish under the MFMAs.
+    struct Opnd {
+        v4i A[7], B[NW][3], E[NW];
+    };
+    auto rdA = [&](const uint8_t(&src)[PSTAGE], int a) {
+        return *reinterpret_cast<const v4i *>(src + wt * SLICE + a * PLANE + off);
+    };
+    auto rdB = [&](const uint8_t(&src)[PSTAGE], int k) {   // k = 3 n + j
+        return *reinterpret_cast<const v4i *>(src + PX_BYTES + k * PLANE + wn * SLICE + off);
+    };
+    auto rdX = [&](const uint8_t(&src)[PSTAGE], int n) {
+        return *reinterpret_cast<const v4i *>(src + XB + n * PLANE + wn * SLICE + off);
+    };
+    auto rd = [&](const uint8_t(&src)[PSTAGE], Opnd &o) {
+#pragma unroll
+        for (int a = 0; a < 7; ++a)
+            o.A[a] = rdA(src, a);
+#pragma unroll
+        for (int n = 0; n < NW; ++n) {
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                o.B[n][j] = rdB(src, 3 * n + j);
+            o.E[n] = rdX(src, n);
+        }
+    };
+    // Step i with operands o (e: its ext bits), leaving the next
+    // step's operands, read from nxt, in the same registers as they come free:
+    // A[a] is read again once plane a's MFMAs are issued.  Step i + 3's DMA into
+    // ldst (el: its ext bits) goes out between the MFMAs too: one wave runs per
+    // SIMD, so its address arithmetic ahead of the MFMAs leaves the matrix core
+    // idle.  The order is fixed by scheduling barriers.
+    auto step = [&](int i, uint32_t e, Opnd &o, const uint8_t(&nxt)[PSTAGE], uint32_t el,
+                    uint8_t(&ldst)[PSTAGE]) {
+        const Src f = src_of(i + 3);
+        constexpr int EVERY = 21 * NW / CPW;
+        if (e) {
+#pragma unroll
+            for (int n = 0; n < NW; ++n)
+                if ((e >> n) & 1u)
+#pragma unroll
+                    for (int a = 0; a < 7; ++a)
+                        mfma_i8(acc, n, a + 1, o.A[a], o.E[n]);
+            if (e & 4u)
+#pragma unroll
+                for (int n = 0; n < NW; ++n) {
+                    const v4i Bx = *reinterpret_cast<const v4i *>(wsrc[n] + src_of(i).w +
+                                                                  wn * SLICE + off);
+#pragma unroll
+                    for (int a = 0; a < 7; ++a)
+                        mfma_i8(acc, n, a, o.A[a], Bx);
+                }
+        }
+        v4i nb[NW][3], a6;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int a = 0; a < 7; ++a) {
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+#pragma unroll
+                for (int n = 0; n < NW; ++n) {
+                    const int m = (a * 3 + j) * NW + n;   // MFMA of the step
+                    mfma_i8(acc, n, a + 2 + j, o.A[a], o.B[n][j]);
+                    // a read or two under the MFMAs of a plane, the last one
+                    // (A[5]) six MFMAs or three from the step's end
+                    if (j == 0 && n == 0) {
+                        if (a < 3 * NW)
+                            nb[a / 3][a % 3] = rdB(nxt, a);
+                        if (a > 0)
+                            o.A[a - 1] = rdA(nxt, a - 1);
+                    }
+                    if (j == 1 && n == 0) {
+                        if (a < NW)
+                            o.E[a] = rdX(nxt, a);
+                        if (a == 5)
+                            a6 = rdA(nxt, 6);
+                    }
+                    if (m % EVERY == EVERY / 2 && m / EVERY < CPW)
+                        dma1(m / EVERY, f, el, ldst);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+        }
+        o.A[6] = a6;
+#pragma unroll
+        for (int n = 0; n < NW; ++n)
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                o.B[n][j] = nb[n][j];
+    };
+    // ext bits of loop steps i .. i + 3, from their bytes in a word
+    auto ext4 = [&](uint32_t v, uint32_t &f0, uint32_t &f1, uint32_t &f2, uint32_t &f3) {
+        const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+        f0 = f & 7u;
+        f1 = (f >> 8) & 7u;
+        f2 = (f >> 16) & 7u;
+        f3 = f >> 24;
+    };
+    auto ext_word = [&](int i) { return *reinterpret_cast<const uint32_t *>(ext + i); };
+    // prologue: steps 0..2 landed (their X chunks are in flight already), step 0
+    // read.  e0..e3: ext bits of the group's steps; en: the next group's word,
+    // read a group ahead.
+    uint32_t e0, e1, e2, e3;
+    ext4(ext_word(0), e0, e1, e2, e3);
+    uint32_t en = ext_word(4);
+    dma(0, e0, s0);
+    dma(1, e1, s1);
+    dma(2, e2, s2);
+    wait_vm<0>();
+    stage_barrier();
+    Opnd o;
+    rd(s0, o);
+    for (int i = 0; i < ns; i += 4) {
+        uint32_t e4, e5, e6, e7;
+        ext4(en, e4, e5, e6, e7);
+        wait_vm<CPW>();
+        stage_barrier();
+        en = ext_word(i + 8);
+        step(i, e0, o, s1, e3, s3);
+        wait_vm<CPW>();
+        stage_barrier();
+        step(i + 1, e1, o, s2, e4, s0);
+        wait_vm<CPW>();
+        stage_barrier();
+        step(i + 2, e2, o, s3, e5, s1);
+        wait_vm<CPW>();
+        stage_barrier();
+        step(i + 3, e3, o, s0, e6, s2);
+        e0 = e4;
+        e1 = e5;
+        e2 = e6;
+        e3 = e7;
+    }
+    wait_vm<0>();   // no DMA in flight when the block gives its LDS back
 }
 
-// grid (ceil(N/64) * ceil(T/64), 1, S) over operands split by k_planes
-// (nsteps k-steps): split z covers steps [z spb, (z + 1) spb).  The block
-// ORs its tiles' masks over its steps; the window is LO = top W plane - 3
-// (clamped to 0..4); a block whose X digits reach plane 7 (or may overflow)
-// or whose W digits leave LO - 1 .. LO + 3 writes nothing and sets
-// redo[block] (else clears it) for k_gemm_i8_full.  S == 1: Y gets the
-// shifted result; S > 1: P[z][t][n] the int128 partial.
+// a * 2^S + c (one v_mad_i64_i32; the compiler takes a shift, a sign
+// extension and two additions)
+template <int S>
+__device__ __forceinline__ int64_t mad_shl(int a, int64_t c)
+{
+    int64_t r;
+    uint64_t cy;
+    asm("v_mad_i64_i32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(cy) : "v"(a), "s"(1 << S), "v"(c));
+    return r;
+}
+
+// Register i of the 11 window digit sums as the 128-bit sum S = sum_r acc[r][i]
+// 256^r (two words; |S| < 2^112): groups of four are exact int64 (|g| < 2^31
+// (1 + 2^8 + 2^16 + 2^24) < 2^56), S = g0 + 2^32 g1 + 2^64 g2 with one carry.
+__device__ __forceinline__ void win_sum128(const v16i (&acc)[11], int i, uint64_t &lo,
+                                           uint64_t &hi)
+{
+    int64_t g[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        g[j] = mad_shl<8>(acc[4 * j + 1][i], (int64_t)acc[4 * j][i]);
+        g[j] = mad_shl<16>(acc[4 * j + 2][i], g[j]);
+        if (j < 2)
+            g[j] = mad_shl<24>(acc[4 * j + 3][i], g[j]);
+    }
+    lo = (uint64_t)g[0] + ((uint64_t)g[1] << 32);
+    const uint64_t carry = lo < (uint64_t)g[0] ? 1u : 0u;
+    hi = (uint64_t)(g[0] >> 63) + (uint64_t)(g[1] >> 32) + carry + (uint64_t)g[2];
+}
+
+// grid (ceil(ceil(N/64) / NW) * ceil(T/64), 1, S) over operands split by
+// k_planes (nsteps k-steps): split z covers steps [z spb, (z + 1) spb), and a
+// block NW row tiles of W.  The block ORs its tiles' masks over its steps;
+// TOP is its W's top plane (at least 4); a block whose X digits reach plane 7
+// (or may overflow) or whose W digits leave TOP - 4 .. TOP writes nothing and
+// sets its tiles' redo flags (else clears them; the flag of a 64 x 64 tile is
+// that of its block in k_gemm_i8_full's numbering).  S == 1: Y gets the shifted
+// result; S > 1: P[z][t][n] the int128 partial.  Row tiles whose planes are
+// shifted (prepared weights) give sums 2^shift too large: exact multiples,
+// shifted back.
+//
+// Two row tiles (NW = 2) halve the X traffic and the barriers per product: a
+// step moves 26 KB for 42 MFMAs a wave, where NW = 1 moves 20 KB for 21.
+//
+// What bounds it: the matrix cores at the clock their power allows.  A loop of
+// nothing but these MFMAs on random digits runs at 3.3 POP/s (4.5-4.9 on
+// zeros); 2048 x 11264 x 2048 takes 22 digit products per Q16.48 MAC here, 2.8
+// POP/s over its 745 us.  With a four-plane window always multiplied (28
+// products), the DMA ahead of the MFMAs and a 64-bit vector address per chunk
+// the call took 991 us on the same card (776 now with the split of X).
+template <int NW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ redo,
            const uint8_t *__restrict__ Xp, const uint32_t *__restrict__ Xm,
            const uint8_t *__restrict__ Wp, const uint32_t *__restrict__ Wm, int T, int N,
            int nsteps, int spb, int cpx)
 {
+    constexpr int PSTAGE = stage_bytes(NW);
     __shared__ __align__(16) uint8_t st0[PSTAGE];
     __shared__ __align__(16) uint8_t st1[PSTAGE];
     __shared__ __align__(16) uint8_t st2[PSTAGE];
     __shared__ __align__(16) uint8_t st3[PSTAGE];
     __shared__ uint32_t red[2][4];
+    // a byte per loop step, and the groups' words a group ahead
+    constexpr int EXT_BYTES = 512;
+    static_assert(MAXK_RUN / MK <= 510 && 256 * 2 == EXT_BYTES, "two steps a thread");
+    __shared__ __align__(4) uint8_t ext[EXT_BYTES + 12];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    int n_tile, t_tile;
-    tile_of(blockIdx.x, (N + MN - 1) / MN, (T + MT - 1) / MT, n_tile, t_tile);
-    const int s0 = (int)blockIdx.z * spb, ns = max(0, min(nsteps, s0 + spb) - s0);
-    uint32_t mx = 0, mw = 0;
-    for (int i = tid; i < ns; i += 256) {
-        mx |= Xm[(size_t)t_tile * nsteps + s0 + i];
-        mw |= Wm[(size_t)n_tile * nsteps + s0 + i];
+    const int nn = (N + MN - 1) / MN, nt = (T + MT - 1) / MT;
+    int n_blk, t_tile;
+    tile_of(blockIdx.x, (nn + NW - 1) / NW, nt, n_blk, t_tile);
+    // a split past the last k-step is empty, at nsteps
+    const int s0 = min((int)blockIdx.z * spb, nsteps), ns = min(nsteps, s0 + spb) - s0;
+    int n_tile[NW];   // past the last row tile: that one again, not stored
+#pragma unroll
+    for (int j = 0; j < NW; ++j)
+        n_tile[j] = min(NW * n_blk + j, nn - 1);
+    // Blocks run in rounds of one per compute unit; each XCD's round holds 8
+    // row blocks x 4 token tiles (tile_of), and the next round's blocks take
+    // the same row blocks with the next token tiles.  Odd rounds walk k
+    // downwards, so they start on the W planes the round before ended on,
+    // which are still in L2.
+    const bool rev = ((((int)blockIdx.x >> 3) / cpx) & 1) != 0;
+    // the masks of loop steps tid and tid + 256 (ns <= 510)
+    uint32_t mx = 0, mw = 0, wk[2][NW];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int i = tid + 256 * u, k = s0 + (rev ? ns - 1 - i : i);
+#pragma unroll
+        for (int j = 0; j < NW; ++j)
+            wk[u][j] = i < ns ? Wm[(size_t)n_tile[j] * nsteps + k] & 0xffffu : 0u;
+        mx |= i < ns ? Xm[(size_t)t_tile * nsteps + k] : 0u;
     }
+    const uint8_t *xsrc = Xp + ((size_t)t_tile * (nsteps + 1) + s0) * 8 * PLANE;
+    planes_first_x(st0, st1, st2, xsrc, ns, nsteps - s0, rev);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int j = 0; j < NW; ++j)
+            mw |= wk[u][j];
     mx = wave_or(mx);
     mw = wave_or(mw);
     if (lane == 0) {
@@ -929,72 +1224,86 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
     __syncthreads();
     mx = (uint32_t)__builtin_amdgcn_readfirstlane((int)(red[0][0] | red[0][1] | red[0][2] | red[0][3]));
     mw = (uint32_t)__builtin_amdgcn_readfirstlane((int)(red[1][0] | red[1][1] | red[1][2] | red[1][3]));
-    const int top = (mw & 0xffu) ? 31 - __builtin_clz(mw & 0xffu) : 3;
-    const int LO = min(max(top - 3, 0), 4);
-    const uint32_t win = ((0x1fu << LO) >> 1) & 0xffu;
+    const int top = max((mw & 0xffu) ? 31 - __builtin_clz(mw & 0xffu) : 0, 4);
+    const uint32_t win = 0x1fu << (top - 4);
     const bool fit = (mx & ~0x7fu) == 0 && (mw & ~win) == 0;
-    if (tid == 0)
-        redo[blockIdx.z * gridDim.x + blockIdx.x] = fit ? 0 : 1;
-    if (!fit)
-        return;   // uniform over the block
+    if (tid < NW && NW * n_blk + tid < nn)
+        redo[blockIdx.z * nn * nt + block_of(NW * n_blk + tid, t_tile, nn, nt)] = fit ? 0 : 1;
+    if (!fit) {
+        wait_vm<0>();   // no DMA in flight when the block gives its LDS back
+        return;         // uniform over the block
+    }
 
-    v16i acc[14];
+    v16i acc[NW][11];
 #pragma unroll
-    for (int d = 0; d < 14; ++d)
-        acc[d] = (v16i){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const uint8_t *xsrc = Xp + ((size_t)t_tile * nsteps + s0) * 8 * PLANE;
-    const uint8_t *wsrc = Wp + ((size_t)n_tile * nsteps + s0) * 8 * PLANE;
-    const ConstMask wm = (ConstMask)(Wm + (size_t)n_tile * nsteps + s0);
-    // Blocks run in rounds of one per compute unit; each XCD's round holds 8
-    // row tiles x 4 token tiles (tile_of), and the next round's blocks take
-    // the same row tiles with the next token tiles.  Odd rounds walk k
-    // downwards, so they start on the W planes the round before ended on,
-    // which are still in L2.
-    const bool rev = ((((int)blockIdx.x >> 3) / cpx) & 1) != 0;
-    // lane l, register i: token 8 (i / 4) + 4 (l / 32) + i % 4, row l % 32;
-    // window LO touches digit sums LO - 1 .. LO + 9 only
+    for (int j = 0; j < NW; ++j)
+#pragma unroll
+        for (int d = 0; d < 11; ++d)
+            acc[j][d] = (v16i){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const uint8_t *wsrc[NW];
+#pragma unroll
+    for (int j = 0; j < NW; ++j)
+        wsrc[j] = Wp + ((size_t)n_tile[j] * nsteps + s0) * 8 * PLANE + (top - 4) * PLANE;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int i = tid + 256 * u;
+        uint32_t b = 0;
+#pragma unroll
+        for (int j = 0; j < NW; ++j) {
+            const uint32_t m = wk[u][j] >> (top - 4);
+            b |= ((m >> 1) & 1u) << j | (m & 1u) << 2;
+        }
+        if (i < EXT_BYTES)
+            ext[i] = (uint8_t)b;
+    }
+    __syncthreads();
+    if (ns > 0)   // an empty split has its X slots' zeros in flight: waited for below
+        planes_pass<NW>(st0, st1, st2, st3, ext, xsrc, wsrc, ns, nsteps - s0, rev, acc);
+    else
+        wait_vm<0>();
+    mfma_settle<NW>(acc);
+    // lane l, register i: token 8 (i / 4) + 4 (l / 32) + i % 4, row l % 32
     const int wt = w >> 1, wn = w & 1;
-    const int n = n_tile * MN + 32 * wn + (lane & 31);
-    auto store = [&](auto d0, auto d1) {
-        if (n >= N)
-            return;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int t = t_tile * MT + 32 * wt + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-            if (t >= T)
-                continue;
-            uint64_t lo, hi;
-            acc_sum128<decltype(d0)::value, decltype(d1)::value>(acc, i, lo, hi);
-            if (gridDim.z == 1) {
-                Y[(size_t)t * N + n] = (int64_t)((hi << 16) | (lo >> 48));
-            } else {
+    for (int j = 0; j < NW; ++j) {
+        const int n = (NW * n_blk + j) * MN + 32 * wn + (lane & 31);
+        const int t0 = t_tile * MT + 32 * wt + 4 * (lane >> 5);
+        const int wsh = (int)((Wm[(size_t)n_tile[j] * nsteps] >> 16) & 7u);
+        const int sh = 48 + wsh - 8 * (top - 4);   // 24 .. 55
+        if (gridDim.z == 1) {
+            int64_t y[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                uint64_t lo, hi;
+                win_sum128(acc[j], i, lo, hi);
+                y[i] = (int64_t)((lo >> sh) | (hi << (64 - sh)));
+            }
+            int64_t *p = Y + (size_t)t0 * N + n;
+            if ((t_tile + 1) * MT <= T && (NW * n_blk + j + 1) * MN <= N) {   // whole tile
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    p[(size_t)(8 * (i >> 2) + (i & 3)) * N] = y[i];
+            } else if (n < N) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (t0 + 8 * (i >> 2) + (i & 3) < T)
+                        p[(size_t)(8 * (i >> 2) + (i & 3)) * N] = y[i];
+            }
+        } else if (n < N) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int t = t0 + 8 * (i >> 2) + (i & 3);
+                if (t >= T)
+                    continue;
+                uint64_t lo, hi;
+                win_sum128(acc[j], i, lo, hi);
+                const q48_i128 u =
+                    (q48_i128)((((q48_u128)hi << 64) | lo) << (8 * (top - 4))) >> wsh;
                 uint64_t *p = P + 2 * (((size_t)blockIdx.z * T + t) * N + n);
-                *reinterpret_cast<ulonglong2 *>(p) = make_ulonglong2(lo, hi);
+                *reinterpret_cast<ulonglong2 *>(p) =
+                    make_ulonglong2((uint64_t)u, (uint64_t)((q48_u128)u >> 64));
             }
         }
-    };
-    using std::integral_constant;
-    switch (LO) {
-    case 0:
-        planes_pass<0>(st0, st1, st2, st3, wm, xsrc, wsrc, ns, rev, acc);
-        store(integral_constant<int, 0>{}, integral_constant<int, 9>{});
-        break;
-    case 1:
-        planes_pass<1>(st0, st1, st2, st3, wm, xsrc, wsrc, ns, rev, acc);
-        store(integral_constant<int, 0>{}, integral_constant<int, 10>{});
-        break;
-    case 2:
-        planes_pass<2>(st0, st1, st2, st3, wm, xsrc, wsrc, ns, rev, acc);
-        store(integral_constant<int, 1>{}, integral_constant<int, 11>{});
-        break;
-    case 3:
-        planes_pass<3>(st0, st1, st2, st3, wm, xsrc, wsrc, ns, rev, acc);
-        store(integral_constant<int, 2>{}, integral_constant<int, 12>{});
-        break;
-    default:
-        planes_pass<4>(st0, st1, st2, st3, wm, xsrc, wsrc, ns, rev, acc);
-        store(integral_constant<int, 3>{}, integral_constant<int, 13>{});
-        break;
     }
 }
 
@@ -1036,8 +1345,9 @@ int q48_launch_gemm_prepare(q48_ctx *c, void *Wp, const int64_t *W, int N, int K
         return Q48_EINVAL;
     uint8_t *p = (uint8_t *)Wp;
     uint32_t *m = (uint32_t *)(p + (size_t)nn * steps * 8 * PLANE);
+    hipLaunchKernelGGL(k_tile_shift, dim3(nn), dim3(1024), 0, c->stream, m, W, N, K, steps);
     hipLaunchKernelGGL(k_planes, dim3(nn * steps), dim3(256), 0, c->stream, p, m, W, N, K,
-                       steps);
+                       steps, steps, 1);
     return (int)hipGetLastError();
 }
 
@@ -1056,7 +1366,7 @@ int q48_launch_gemm_i8(q48_ctx *c, int64_t *Y, const int64_t *W, const int64_t *
     // N >= 2048 faster by 7-39%, N = 256 slower by 5-22%, T = 128 even when
     // W is split in the call); with W prepared it wins from 2 tokens, where
     // the GEMM streams W and the planes hold 5 of its 8 bytes per element
-    const bool fits = (size_t)max(nt, nn) * steps <= 0x7fffffff;
+    const bool fits = (size_t)max(nt, nn) * (steps + 1) <= 0x7fffffff;
     const bool planes =
         fits && (kernel == Q48_GEMM_I8_PLANES ||
                  (kernel != Q48_GEMM_I8_FUSED && T >= (Wpre ? 2 : 256) && N >= 1024));
@@ -1066,7 +1376,7 @@ int q48_launch_gemm_i8(q48_ctx *c, int64_t *Y, const int64_t *W, const int64_t *
     // (planes path) X and W digit planes and their masks
     const size_t flags = al((size_t)nb * S * sizeof(int));
     const size_t part = S > 1 ? 16 * (size_t)S * T * N : 0;
-    const size_t xpl = planes ? (size_t)nt * steps * 8 * PLANE : 0;
+    const size_t xpl = planes ? (size_t)nt * (steps + 1) * 8 * PLANE : 0;
     const size_t wpl = wsplit ? (size_t)nn * steps * 8 * PLANE : 0;
     const size_t xms = planes ? al((size_t)nt * steps * 4) : 0;
     const size_t wms = wsplit ? al((size_t)nn * steps * 4) : 0;
@@ -1082,18 +1392,32 @@ int q48_launch_gemm_i8(q48_ctx *c, int64_t *Y, const int64_t *W, const int64_t *
     if (planes) {
         uint8_t *Xp = (uint8_t *)(ws + flags + part), *Wp = Xp + xpl;
         uint32_t *Xm = (uint32_t *)(Wp + wpl), *Wm = (uint32_t *)((char *)Xm + xms);
-        hipLaunchKernelGGL(k_planes, dim3(nt * steps), dim3(256), 0, c->stream, Xp, Xm, X, T, K,
-                           steps);
+        hipLaunchKernelGGL(k_planes, dim3(nt * (steps + 1)), dim3(256), 0, c->stream, Xp, Xm,
+                           X, T, K, steps, steps + 1, 0);
         if (Wpre) {
             // planes from q48_launch_gemm_prepare: masks after the planes
             Wp = (uint8_t *)Wpre;
             Wm = (uint32_t *)(Wp + (size_t)nn * steps * 8 * PLANE);
         } else {
             hipLaunchKernelGGL(k_planes, dim3(nn * steps), dim3(256), 0, c->stream, Wp, Wm, W, N,
-                               K, steps);
+                               K, steps, steps, 0);
         }
-        hipLaunchKernelGGL(k_gemm_i8p, grid, dim3(256), 0, c->stream, Y, P, redo, Xp, Xm, Wp, Wm,
-                           T, N, steps, spb, max(1, c->cu_count / 8));
+        // one or two row tiles a block, by rounds of blocks over the compute
+        // units: a block of two takes 1.93 times one of one (2048 x 11264 x
+        // 2048: 22 rounds in 806 us, 11 in 776), so two win where they need
+        // half the rounds (or a little over half, with many), and lose where
+        // the last round is emptier (2048 x 2048, 1500 tokens: 3 rounds 121
+        // us, 2 rounds 136).  Split K keeps one: its runs are short, and the
+        // part that fills the device is what it is for (128 tokens x 2560 x
+        // 2048: 39.0 against 41.6 us).
+        const int cu = c->cu_count, cpx = max(1, cu / 8), nb2 = (nn + 1) / 2 * nt;
+        const int rounds1 = (nb + cu - 1) / cu, rounds2 = (nb2 + cu - 1) / cu;
+        if (S == 1 && 29 * rounds2 <= 15 * rounds1)
+            hipLaunchKernelGGL(k_gemm_i8p<2>, dim3(nb2, 1, 1), dim3(256), 0, c->stream, Y, P,
+                               redo, Xp, Xm, Wp, Wm, T, N, steps, spb, cpx);
+        else
+            hipLaunchKernelGGL(k_gemm_i8p<1>, grid, dim3(256), 0, c->stream, Y, P, redo, Xp, Xm,
+                               Wp, Wm, T, N, steps, spb, cpx);
     } else if (vec) {
         hipLaunchKernelGGL((k_gemm_i8<true>), grid, dim3(256), 0, c->stream, Y, P, redo, W, X, T,
                            N, K, spb);
