@@ -678,6 +678,31 @@ __device__ __forceinline__ int64_t q48_safe_exp(int64_t x)
     return q48_exp_small(x);
 }
 
+// fp_safe_exp(-u) for the softmax's u = max - score, 0 <= u < 2^63 (no wrapped
+// difference): q48_safe_exp with one sign and no branch.  Arguments past the
+// clamp run at it and give 0; q48_recip's quotient without its fallback (its
+// estimate is within the bounds there for every r = e^u, 0 <= u <= 10).
+__device__ __forceinline__ int64_t q48_exp_neg(uint64_t u)
+{
+    const uint64_t lim = (uint64_t)10 << 48;
+    const bool in = u <= lim;
+    const uint64_t m = in ? u : lim;
+    double h = __builtin_bit_cast(double, 0x4330000000000000ull + (uint64_t)Q48_ONE + (m >> 14));
+#pragma unroll
+    for (int k = 0; k < 12; ++k) {
+        const double y = __builtin_fma(h, 0x1p-24, -0x1p28);
+        h = __builtin_fma(y, y, 0x1p52);
+    }
+    const uint64_t r = (uint64_t)q48_usqr((uint64_t)q48_usqr(q48_word_m52(h)));
+    const double rd = (double)r;
+    double y = __builtin_amdgcn_rcp(rd);
+    y = __builtin_fma(y, __builtin_fma(-rd, y, 1.0), y);
+    y = __builtin_fma(y, __builtin_fma(-rd, y, 1.0), y);
+    const uint64_t q0 = q48_word_m52(__builtin_fma(y, 0x1p96, 0x1p52 - 0.5));
+    const uint64_t rem = (uint64_t)0 - q0 * r;
+    return in ? (int64_t)(q0 + (rem >= r ? 1 : 0)) : 0;
+}
+
 // fp_log, fp_math.h:752-773
 __device__ __forceinline__ int64_t q48_log(int64_t x)
 {

@@ -53,6 +53,42 @@ __device__ __forceinline__ void digits4(const uint64_t (&v)[4], uint32_t (&w)[8]
     w[7] = hi[3];
 }
 
+// a 2^S + c in one v_mad_i64_i32: with the factor known, the compiler takes a
+// shift, a sign extension and two additions.  (Not written as assembly: a is
+// often an MFMA result, whose wait states the compiler inserts only before
+// instructions it knows.)
+template <int S>
+__device__ __forceinline__ int64_t mad_shl(int a, int64_t c)
+{
+    int m = 1 << S;
+    asm("" : "+s"(m));
+    return (int64_t)a * (int64_t)m + c;
+}
+
+// bits 48..111 of sum_d 256^d q[d][i] + c over the 14 digit-product
+// accumulators, c the 128-bit correction: four groups of digit sums, each an
+// exact int64 that starts from c's word (|q| < 2^31, so a group stays below
+// 2^56), joined by their signed high words; 25 operations.
+template <typename V>
+__device__ __forceinline__ int64_t digits_shr48(const V (&q)[14], int i, q48_u128 c)
+{
+    int64_t g[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        g[j] = mad_shl<0>(q[4 * j][i], (int64_t)(uint32_t)(c >> (32 * j)));
+        g[j] = mad_shl<8>(q[4 * j + 1][i], g[j]);
+        if (j < 3) {
+            g[j] = mad_shl<16>(q[4 * j + 2][i], g[j]);
+            g[j] = mad_shl<24>(q[4 * j + 3][i], g[j]);
+        }
+        if (j > 0)
+            g[j] += g[j - 1] >> 32;
+    }
+    const uint32_t w1 = (uint32_t)g[1], w2 = (uint32_t)g[2], w3 = (uint32_t)g[3];
+    return (int64_t)(((uint64_t)__builtin_amdgcn_alignbit(w3, w2, 16) << 32) |
+                     __builtin_amdgcn_alignbit(w2, w1, 16));
+}
+
 // sum_d 256^d q[d][i] (int128) of 14 digit-product accumulators
 __device__ __forceinline__ q48_u128 digits_total(const v4i (&q)[14], int i)
 {

@@ -881,22 +881,22 @@ __device__ __forceinline__ void mfma_i8(v16i (&acc)[NW][11], int n, int r, const
     else
         mfma_asm<false>(acc[n][r], a, b);
 }
-// The sums after mfma_asm: an MFMA's result may be read by other vector
+// The sums after the k loop: an MFMA's result may be read by other vector
 // instructions only after its passes (at most 18 wait states), which the
-// compiler does not know of here; what reads a sum depends on this.
+// compiler adds before the instructions it knows but not around mfma_asm and
+// mad_shl_asm; what reads a sum depends on this.
 template <int NW>
 __device__ __forceinline__ void mfma_settle(v16i (&acc)[NW][11])
 {
-    if constexpr (NW > 1) {
-        asm volatile("s_nop 15\n\ts_nop 15"
-                     : "+a"(acc[0][0]), "+a"(acc[0][1]), "+a"(acc[0][2]), "+a"(acc[0][3]),
-                       "+a"(acc[0][4]), "+a"(acc[0][5]), "+a"(acc[0][6]), "+a"(acc[0][7]),
-                       "+a"(acc[0][8]), "+a"(acc[0][9]), "+a"(acc[0][10]));
+    asm volatile("s_nop 15\n\ts_nop 15"
+                 : "+a"(acc[0][0]), "+a"(acc[0][1]), "+a"(acc[0][2]), "+a"(acc[0][3]),
+                   "+a"(acc[0][4]), "+a"(acc[0][5]), "+a"(acc[0][6]), "+a"(acc[0][7]),
+                   "+a"(acc[0][8]), "+a"(acc[0][9]), "+a"(acc[0][10]));
+    if constexpr (NW > 1)
         asm volatile(""
                      : "+a"(acc[1][0]), "+a"(acc[1][1]), "+a"(acc[1][2]), "+a"(acc[1][3]),
                        "+v"(acc[1][4]), "+v"(acc[1][5]), "+v"(acc[1][6]), "+v"(acc[1][7]),
                        "+v"(acc[1][8]), "+v"(acc[1][9]), "+v"(acc[1][10]));
-    }
 }
 
 // The X chunks of slots 0 .. XSLOTS - 1 (which hold no W) of the loop's steps
@@ -1115,10 +1115,10 @@ __device__ __forceinline__ void planes_pass(uint8_t (&s0)[stage_bytes(NW)],
     wait_vm<0>();   // no DMA in flight when the block gives its LDS back
 }
 
-// a * 2^S + c (one v_mad_i64_i32; the compiler takes a shift, a sign
-// extension and two additions)
+// mad_shl as assembly, for the settled sums: the compiler's own form of it here
+// spills in k_gemm_i8p<2>.
 template <int S>
-__device__ __forceinline__ int64_t mad_shl(int a, int64_t c)
+__device__ __forceinline__ int64_t mad_shl_asm(int a, int64_t c)
 {
     int64_t r;
     uint64_t cy;
@@ -1135,10 +1135,10 @@ __device__ __forceinline__ void win_sum128(const v16i (&acc)[11], int i, uint64_
     int64_t g[3];
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-        g[j] = mad_shl<8>(acc[4 * j + 1][i], (int64_t)acc[4 * j][i]);
-        g[j] = mad_shl<16>(acc[4 * j + 2][i], g[j]);
+        g[j] = mad_shl_asm<8>(acc[4 * j + 1][i], (int64_t)acc[4 * j][i]);
+        g[j] = mad_shl_asm<16>(acc[4 * j + 2][i], g[j]);
         if (j < 2)
-            g[j] = mad_shl<24>(acc[4 * j + 3][i], g[j]);
+            g[j] = mad_shl_asm<24>(acc[4 * j + 3][i], g[j]);
     }
     lo = (uint64_t)g[0] + ((uint64_t)g[1] << 32);
     const uint64_t carry = lo < (uint64_t)g[0] ? 1u : 0u;

@@ -236,6 +236,10 @@ k_pfa(int64_t *__restrict__ out, const int64_t *__restrict__ QKV,
 
     // phase 1: lane holds position j0 + rl of rows 4 kq + i
     int64_t mx[4] = {INT64_MIN, INT64_MIN, INT64_MIN, INT64_MIN};
+    uint32_t far = 0;   // bit 31: a score outside [-2^62, 2^62)
+    // a scale that is a power of two (head_dim 64: 2^45) multiplies by a shift
+    const bool pow2 = scale > 0 && scale <= Q48_ONE && (scale & (scale - 1)) == 0;
+    const int sshr = 48 - (63 - __builtin_clzll((uint64_t)(scale > 0 ? scale : 1)));
     {
         const uint8_t *kd = KD + (size_t)kh * 8 * Ppad * HDP;
         const uint64_t *ck = CK + 2 * (size_t)kh * Ppad;
@@ -265,9 +269,10 @@ k_pfa(int64_t *__restrict__ out, const int64_t *__restrict__ QKV,
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int m = 4 * kq + i;
-                const q48_u128 tot = digits_total(acc, i) + cq[m] + ckj;
-                const int64_t s = q48_mul((int64_t)(tot >> 48), scale);
+                const int64_t dot = digits_shr48(acc, i, cq[m] + ckj);
+                const int64_t s = pow2 ? dot >> sshr : q48_mul(dot, scale);
                 sc[(size_t)m * J + j] = s;
+                far |= (uint32_t)((uint64_t)s >> 32) + 0x40000000u;
                 if (m < nrow && j <= p0 + t0 + m)
                     mx[i] = s > mx[i] ? s : mx[i];
             }
@@ -280,9 +285,13 @@ k_pfa(int64_t *__restrict__ out, const int64_t *__restrict__ QKV,
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             mxs[w][4 * kq + i] = mx[i];
+    if (far & 0x80000000u)
+        atomicOr(&form, 4);
     __syncthreads();
 
-    // phase 2: row r = tid / 16, positions tid % 16 + 16 k
+    // phase 2: row r = tid / 16, positions tid % 16 + 16 k.  With every score
+    // (of any tile position, masked ones too) within 2^62 of zero no difference
+    // to the maximum wraps and q48_exp_neg serves; else q48_safe_exp.
     {
         const int r = tid >> 4, jj = tid & 15;
         int64_t sum = 0;
@@ -294,20 +303,32 @@ k_pfa(int64_t *__restrict__ out, const int64_t *__restrict__ QKV,
                 m = mxs[u][r] > m ? mxs[u][r] : m;
             const int S = p0 + t0 + r + 1;
             int64_t *srow = sc + (size_t)r * J;
-            auto ex = [&](int j) {
-                const int64_t e = q48_safe_exp((int64_t)((uint64_t)srow[j] - (uint64_t)m));
-                srow[j] = e;
-                odd |= (uint64_t)e > (uint64_t)Q48_ONE ? 1 : 0;
-                return e;
-            };
-            int j = jj;
-            for (; j + 48 < S; j += 64) {
-                const int64_t e0 = ex(j), e1 = ex(j + 16), e2 = ex(j + 32), e3 = ex(j + 48);
-                sum = (int64_t)((uint64_t)sum + (uint64_t)e0 + (uint64_t)e1 + (uint64_t)e2 +
-                                (uint64_t)e3);
+            if ((form & 4) == 0) {
+                auto ex = [&](int64_t s) { return q48_exp_neg((uint64_t)m - (uint64_t)s); };
+                int j = jj;
+                for (; j + 48 < S; j += 64) {
+                    const int64_t s0 = srow[j], s1 = srow[j + 16], s2 = srow[j + 32],
+                                  s3 = srow[j + 48];
+                    const int64_t e0 = ex(s0), e1 = ex(s1), e2 = ex(s2), e3 = ex(s3);
+                    srow[j] = e0;
+                    srow[j + 16] = e1;
+                    srow[j + 32] = e2;
+                    srow[j + 48] = e3;
+                    sum += e0 + e1 + e2 + e3;   // at most 16320 ONE
+                }
+                for (; j < S; j += 16) {
+                    const int64_t e = ex(srow[j]);
+                    srow[j] = e;
+                    sum += e;
+                }
+            } else {
+                for (int j = jj; j < S; j += 16) {
+                    const int64_t e = q48_safe_exp((int64_t)((uint64_t)srow[j] - (uint64_t)m));
+                    srow[j] = e;
+                    odd |= (uint64_t)e > (uint64_t)Q48_ONE ? 1 : 0;
+                    sum = (int64_t)((uint64_t)sum + (uint64_t)e);
+                }
             }
-            for (; j < S; j += 16)
-                sum = (int64_t)((uint64_t)sum + (uint64_t)ex(j));
         }
         sum = (int64_t)group_sum64<16>((uint64_t)sum);
         if (jj == 0)
@@ -325,7 +346,7 @@ k_pfa(int64_t *__restrict__ out, const int64_t *__restrict__ QKV,
     // exact, at least ONE, and its weights add up to at most ONE; every value
     // of the span is in [-2^51, 2^51).  2: the same weights, larger values.
     // Bit 0: weights of any kind.
-    const int vform = form;
+    const int vform = form & 3;
     const int Smax = p0 + t0 + nrow;
     const size_t kvd = (size_t)n_kv * HD;
     const int64_t *vraw = vcache + (size_t)kh * HD;
