@@ -631,7 +631,7 @@ int q48_rmsnorm_gemv(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
 {
     if (!c || bad_ptrs(y, W, x) || !norm_w || M <= 0 || K <= 0 || M > kMaxDim || K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v2_ok(W, K)) {
+    if (q48_gemv_v5_ok(M, K)) {
         int prc;
         q48_ctx::ProfRec *r = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -651,7 +651,7 @@ int q48_gemv_residual(q48_ctx *c, int64_t *acc, const int64_t *W, const int64_t 
 {
     if (!c || bad_ptrs(acc, W, x) || M <= 0 || K <= 0 || M > kMaxDim || K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v2_ok(W, K)) {
+    if (q48_gemv_v5_ok(M, K)) {
         int prc;
         q48_ctx::ProfRec *r = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -672,7 +672,7 @@ int q48_rmsnorm_gemv_swiglu(q48_ctx *c, int64_t *out, const int64_t *Wgu, const 
     if (!c || bad_ptrs(out, Wgu, x) || !norm_w || ffn <= 0 || K <= 0 || ffn > kMaxDim / 2 ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v2_ok(Wgu, K)) {
+    if (q48_gemv_v5_ok(2 * ffn, K)) {
         int prc;
         q48_ctx::ProfRec *r = prof_begin(c, gemv_bytes(2 * ffn, K, ffn), &prc);
         if (prc)
@@ -903,7 +903,7 @@ int q48_norm_gemv(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
     if (!c || bad_ptrs(y, W, x) || !norm_w || !r || M <= 0 || K <= 0 || M > kMaxDim ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v2_ok(W, K)) {
+    if (q48_gemv_v5_ok(M, K)) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -925,7 +925,7 @@ int q48_norm_gemv_swiglu(q48_ctx *c, int64_t *out, const int64_t *Wgu, const int
     if (!c || bad_ptrs(out, Wgu, x) || !norm_w || !r || ffn <= 0 || K <= 0 ||
         ffn > kMaxDim / 2 || K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v2_ok(Wgu, K)) {
+    if (q48_gemv_v5_ok(2 * ffn, K)) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(2 * ffn, K, ffn), &prc);
         if (prc)
@@ -949,7 +949,7 @@ int q48_gemv_residual_rms(q48_ctx *c, int64_t *acc, const int64_t *W, const int6
     if (!c || bad_ptrs(acc, W, x) || !r_out || M <= 0 || K <= 0 || M > kMaxDim ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v2_ok(W, K)) {
+    if (q48_gemv_v5_ok(M, K)) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -1000,7 +1000,7 @@ int q48_norm_gemv_stats(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t 
     if (!c || bad_ptrs(y, W, x) || !norm_w || !stats || M <= 0 || K <= 0 || M > kMaxDim ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v2_ok(W, K)) {
+    if (q48_gemv_v5_ok(M, K)) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -1019,7 +1019,7 @@ int q48_norm_gemv_swiglu_stats(q48_ctx *c, int64_t *out, const int64_t *Wgu, con
     if (!c || bad_ptrs(out, Wgu, x) || !norm_w || !stats || ffn <= 0 || K <= 0 ||
         ffn > kMaxDim / 2 || K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v2_ok(Wgu, K)) {
+    if (q48_gemv_v5_ok(2 * ffn, K)) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(2 * ffn, K, ffn), &prc);
         if (prc)
@@ -1037,7 +1037,7 @@ int q48_gemv_residual_stats(q48_ctx *c, int64_t *acc, const int64_t *W, const in
 {
     if (!c || bad_ptrs(acc, W, x) || !stats || M <= 0 || K <= 0 || M > kMaxDim || K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v2_ok(W, K)) {
+    if (q48_gemv_v5_ok(M, K)) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)

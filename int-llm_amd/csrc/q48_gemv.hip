@@ -19,9 +19,8 @@
 //     ws += w      (mod 2^64)
 // then S = a0 + 2^64 c0 + 2^32 a1 + 2^96 c1 + 2^64 a2 - 2^63 (ws + xs).
 //
-// GEMV layout: one wavefront per output row (64 lanes x 16 B = 1 KiB per
-// load instruction, fully coalesced), x staged once per block in LDS in
-// flipped form, rows-per-block waves sharing it; 128-bit cross-lane sum.
+// GEMV layout (k_gemv_d): wavefronts along a row (64 lanes x 16 B = 1 KiB per
+// load instruction, fully coalesced), 128-bit cross-lane sum.
 #include "q48_internal.h"
 
 namespace {
@@ -61,89 +60,95 @@ __device__ __forceinline__ q48_u128 acc_value(const LimbAcc &A)
     return S;
 }
 
-constexpr int KCHUNK = 4096;   // x elements staged per pass (32 KiB LDS)
-
-// RPB waves per block, one row per wave.  VEC = 2: 16-byte loads (K even,
-// W 16-byte aligned); VEC = 1: 8-byte loads (any K).
-template <int RPB, int VEC>
-__global__ __launch_bounds__(64 * RPB) void k_gemv(int64_t *__restrict__ y,
-                                                   const int64_t *__restrict__ W,
-                                                   const int64_t *__restrict__ x,
-                                                   int M, int K)
+// k_gemv_d: any K and 8-byte alignment.  S waves share a row (1, 2, 4 or 8: 8 / S
+// rows a block), or a wave takes RW rows (S = 1).  A wave's segment streams as
+// 1 KB tiles (lane l: elements 2 l, 2 l + 1; 16-byte loads, which take any dword
+// alignment, so odd K costs nothing), UNR of each row in flight together with
+// the same elements of x from the cache: nothing is staged and no barrier comes
+// before the loads, at the price of x read once per wave.  The segment's last,
+// partial tile goes out with the first batch.
+template <int S, int UNR, int RW>
+__global__ __launch_bounds__(512) void k_gemv_d(int64_t *__restrict__ y,
+                                               const int64_t *__restrict__ W,
+                                               const int64_t *__restrict__ x, int M, int K,
+                                               int seg)
 {
-    __shared__ __align__(16) uint64_t xs[KCHUNK];
-    __shared__ uint64_t xsum_w[RPB];
+    static_assert(S == 1 || RW == 1, "rows of a wave or waves of a row");
+    typedef unsigned long long v2u __attribute__((ext_vector_type(2), aligned(8)));
+    constexpr int NW = 8, RB = NW * RW / S;
+    __shared__ uint64_t part[NW * RW][2];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row = (int)blockIdx.x * RB + (S > 1 ? wave / S : wave * RW);
+    const int k0 = min((wave % S) * seg, K), kn = row < M ? min(seg, K - k0) : 0;
+    const int nt = kn >> 7, rem = kn & 127;
+    const int64_t *xr = x + k0, *wr[RW];
+#pragma unroll
+    for (int r = 0; r < RW; ++r)   // rows past the end: the last again, not stored
+        wr[r] = W + (size_t)min(row + r, M - 1) * K + k0;
 
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int row = blockIdx.x * RPB + wave;
-    const bool active = row < M;
-    const int64_t *wr = W + (size_t)(active ? row : 0) * (size_t)K;
-
-    LimbAcc A = {0, 0, 0, 0, 0, 0};
+    LimbAcc A[RW];
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+        A[r] = {0, 0, 0, 0, 0, 0};
     uint64_t xsum = 0;
-
-    for (int k0 = 0; k0 < K; k0 += KCHUNK) {
-        const int kc = min(KCHUNK, K - k0);
-        __syncthreads();
-        for (int j = tid; j < kc; j += 64 * RPB) {
-            uint64_t v = (uint64_t)x[k0 + j];
-            xs[j] = v ^ 0x8000000000000000ull;
-            xsum += v;
-        }
-        __syncthreads();
-        if (active) {
-            if (VEC == 2) {
-                const ulonglong2 *w2 = reinterpret_cast<const ulonglong2 *>(wr + k0);
-                const uint4 *x4 = reinterpret_cast<const uint4 *>(xs);
-                const int np = kc >> 1;
-                int p = lane;
-                for (; p + 192 < np; p += 256) {
-                    ulonglong2 wa = w2[p], wb = w2[p + 64], wc = w2[p + 128], wd = w2[p + 192];
-                    uint4 xa = x4[p], xb = x4[p + 64], xc = x4[p + 128], xd = x4[p + 192];
-                    mac_flip(A, xa.x, xa.y, wa.x);
-                    mac_flip(A, xa.z, xa.w, wa.y);
-                    mac_flip(A, xb.x, xb.y, wb.x);
-                    mac_flip(A, xb.z, xb.w, wb.y);
-                    mac_flip(A, xc.x, xc.y, wc.x);
-                    mac_flip(A, xc.z, xc.w, wc.y);
-                    mac_flip(A, xd.x, xd.y, wd.x);
-                    mac_flip(A, xd.z, xd.w, wd.y);
+    auto mac = [&](LimbAcc &a, uint64_t xv, uint64_t wv) {
+        mac_flip(a, (uint32_t)xv, (uint32_t)(xv >> 32) ^ 0x80000000u, wv);
+    };
+    // the partial tile: elements 2 l and 2 l + 1 where they exist (others
+    // multiply 0 by 0, which touches bits 126 and 127 only)
+    uint64_t te[RW][2], xe[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const bool in = 2 * lane + e < rem;
+        xe[e] = in ? (uint64_t)xr[128 * nt + 2 * lane + e] : 0;
+#pragma unroll
+        for (int r = 0; r < RW; ++r)
+            te[r][e] = in ? (uint64_t)wr[r][128 * nt + 2 * lane + e] : 0;
+    }
+    const v2u *x2 = reinterpret_cast<const v2u *>(xr) + lane;
+    for (int t0 = 0; t0 < nt; t0 += UNR) {
+        v2u wv[RW][UNR], xv[UNR];
+#pragma unroll
+        for (int u = 0; u < UNR; ++u)
+#pragma unroll
+            for (int r = 0; r < RW; ++r)
+                wv[r][u] = __builtin_nontemporal_load(reinterpret_cast<const v2u *>(wr[r]) + lane +
+                                                      64 * min(t0 + u, nt - 1));
+#pragma unroll
+        for (int u = 0; u < UNR; ++u)
+            xv[u] = x2[64 * min(t0 + u, nt - 1)];
+#pragma unroll
+        for (int u = 0; u < UNR; ++u)
+            if (t0 + u < nt) {
+#pragma unroll
+                for (int r = 0; r < RW; ++r) {
+                    mac(A[r], xv[u].x, wv[r][u].x);
+                    mac(A[r], xv[u].y, wv[r][u].y);
                 }
-                for (; p < np; p += 64) {
-                    ulonglong2 wa = w2[p];
-                    uint4 xa = x4[p];
-                    mac_flip(A, xa.x, xa.y, wa.x);
-                    mac_flip(A, xa.z, xa.w, wa.y);
-                }
-            } else {
-                const uint2 *x2 = reinterpret_cast<const uint2 *>(xs);
-                for (int j = lane; j < kc; j += 64) {
-                    uint64_t wv = (uint64_t)wr[k0 + j];
-                    uint2 xa = x2[j];
-                    mac_flip(A, xa.x, xa.y, wv);
-                }
+                xsum += xv[u].x + xv[u].y;
             }
+    }
+    xsum += xe[0] + xe[1];
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+        mac(A[r], xe[0], te[r][0]);
+        mac(A[r], xe[1], te[r][1]);
+        A[r].ws += xsum;   // the corrections of x and w add up alike
+        const q48_u128 v = q48_wave_sum128(acc_value(A[r]));
+        if (lane == 0) {
+            part[wave * RW + r][0] = (uint64_t)v;
+            part[wave * RW + r][1] = (uint64_t)(v >> 64);
         }
     }
-
-    // sum of x over the whole row (shared by every row of the block)
-    xsum = (uint64_t)q48_wave_sum64((int64_t)xsum);
-    if (lane == 0)
-        xsum_w[wave] = xsum;
     __syncthreads();
-    if (!active)
-        return;
-    uint64_t xtot = 0;
+    if (tid < RB && (int)blockIdx.x * RB + tid < M) {
+        q48_u128 T = 0;
 #pragma unroll
-    for (int w = 0; w < RPB; ++w)
-        xtot += xsum_w[w];
-
-    q48_u128 S = q48_wave_sum128(acc_value(A));
-    S -= (q48_u128)xtot << 63;
-    if (lane == 0)
-        y[row] = (int64_t)((q48_i128)S >> 48);
+        for (int u = 0; u < S; ++u)
+            T += ((q48_u128)part[tid * S + u][1] << 64) | part[tid * S + u][0];
+        y[(int)blockIdx.x * RB + tid] = (int64_t)((q48_i128)T >> 48);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -209,7 +214,9 @@ template <int WT>
 __device__ __forceinline__ ulonglong2 ld_wtile(const ulonglong2 *p)
 {
     if constexpr (WT == 0) {
-        typedef unsigned long long v2u __attribute__((ext_vector_type(2)));
+        // 16 bytes of a row that may start on 8 (odd K, or W itself): a global
+        // load takes any dword alignment
+        typedef unsigned long long v2u __attribute__((ext_vector_type(2), aligned(8)));
         const v2u v = __builtin_nontemporal_load(reinterpret_cast<const v2u *>(p));
         return make_ulonglong2(v.x, v.y);
     } else {
@@ -509,13 +516,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
                     [&](int t) { return xw + 3 * (64 * t + 8 * l8); });
         }
     } else {
-        // the kn % 16 elements (even) of the segment's end, one pair per lane
-        if (2 * l8 < (kn & 15)) {
-            const ulonglong2 w1 = w2[nt * 8];
-            const uint32_t *p = xl + 48 * nt;
-            mac6(A, p[0], p[1], p[2], w1.x);
-            mac6(A, p[3], p[4], p[5], w1.y);
-        }
+        // the kn % 16 elements of the segment's end, one pair per lane (the
+        // last lane one element when K is odd)
+        const uint64_t *w1 = reinterpret_cast<const uint64_t *>(w2 + nt * 8);
+        const uint32_t *p = xl + 48 * nt;
+        if (2 * l8 < (kn & 15))
+            mac6(A, p[0], p[1], p[2], w1[0]);
+        if (2 * l8 + 1 < (kn & 15))
+            mac6(A, p[3], p[4], p[5], w1[1]);
         S = acc6_value(A);
     }
     S = q48_sum8_u128(S);
@@ -1221,7 +1229,8 @@ static int launch_v4(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
     }
     // K = 2048 and K = 5632 (every wave: 16 or 44 whole tiles) take the
     // unrolled rotating pipeline; other K the batched loop
-    const bool al = ((uintptr_t)x & 15) == 0 && (PRO == 0 || ((uintptr_t)norm_w & 15) == 0) &&
+    const bool al = (((uintptr_t)W | (uintptr_t)x) & 15) == 0 &&
+                    (PRO == 0 || ((uintptr_t)norm_w & 15) == 0) &&
                     (PRO != 3 || ((uintptr_t)r_in & 15) == 0);
     // more row groups than two rounds of blocks: the persistent form
     if constexpr ((PRO == 0 || PRO == 3) && (EPI == 0 || EPI == 2)) {
@@ -1467,6 +1476,11 @@ bool q48_gemv_v2_ok(const int64_t *W, int K)
     return K % 2 == 0 && K <= V2_MAX_K && (((uintptr_t)W & 15) == 0);
 }
 
+// The same kernel on any K and any 8-byte aligned W (its idle waves read two
+// elements of W, so W must hold two): odd K rows start on 8 bytes, and their
+// 16-byte loads go out unaligned.
+bool q48_gemv_v5_ok(int M, int K) { return K <= V2_MAX_K && (M > 1 || K > 1); }
+
 int q48_launch_gemv_fused(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
                           const int64_t *norm_w, const int64_t *r_in, int64_t *r_out, int M,
                           int K, int pro, int epi)
@@ -1587,22 +1601,32 @@ int q48_launch_rms_apply(q48_ctx *c, int64_t *out, const int64_t *x, const int64
 int q48_launch_gemv(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
                     int M, int K)
 {
-    if (q48_gemv_v2_ok(W, K))
+    // the decode kernel where its tiles come out whole, the direct one
+    // elsewhere (us, direct against k_gemv_v5's batched loop: 1376 x 256 4.6 /
+    // 5.5, 4096 x 4096 24.9 / 28.5, 64 x 8191 5.7 / 22.6, 5632 x 1999 19.6 /
+    // 21.9; but 1031 x 2048 7.4 / 5.7 with whole tiles)
+    if ((K == 2048 || K == 5632) && (((uintptr_t)W | (uintptr_t)x) & 15) == 0)
         return launch_v4<0, 0>(c, y, W, x, nullptr, nullptr, nullptr, M, K);
-    const bool vec = (K % 2 == 0) && (((uintptr_t)W & 15) == 0);
-    if (M >= 1024) {
-        dim3 grid((M + 7) / 8);
-        if (vec)
-            hipLaunchKernelGGL((k_gemv<8, 2>), grid, dim3(512), 0, c->stream, y, W, x, M, K);
-        else
-            hipLaunchKernelGGL((k_gemv<8, 1>), grid, dim3(512), 0, c->stream, y, W, x, M, K);
-    } else {
-        dim3 grid((M + 3) / 4);
-        if (vec)
-            hipLaunchKernelGGL((k_gemv<4, 2>), grid, dim3(256), 0, c->stream, y, W, x, M, K);
-        else
-            hipLaunchKernelGGL((k_gemv<4, 1>), grid, dim3(256), 0, c->stream, y, W, x, M, K);
-    }
+    // waves per row: until 2048 waves (8 a compute unit) or one tile each;
+    // many short rows: four a wave, for the loads in flight and x read once
+    int S = 1;
+    while (S < 8 && (size_t)M * S < 2048 && K / (2 * S) >= 128)
+        S *= 2;
+    const int seg = S == 1 ? K : ((K + S - 1) / S + 1) & ~1;
+    auto go = [&](auto kern, int rows) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)((M + rows - 1) / rows)), dim3(512), 0, c->stream,
+                           y, W, x, M, K, seg);
+    };
+    if (S == 1 && K < 512 && M >= 8192)
+        go(k_gemv_d<1, 2, 4>, 32);
+    else if (S == 1)
+        go(k_gemv_d<1, 8, 1>, 8);
+    else if (S == 2)
+        go(k_gemv_d<2, 8, 1>, 4);
+    else if (S == 4)
+        go(k_gemv_d<4, 8, 1>, 2);
+    else
+        go(k_gemv_d<8, 8, 1>, 1);
     return (int)hipGetLastError();
 }
 

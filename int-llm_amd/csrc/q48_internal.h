@@ -88,6 +88,7 @@ uint64_t *q48_scratch_attg_count(int device);
 int q48_launch_gemv(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
                     int M, int K);
 bool q48_gemv_v2_ok(const int64_t *W, int K);
+bool q48_gemv_v5_ok(int M, int K);
 // pro: 0 none, 1 rmsnorm(x, norm_w) computed in every block, 2 with r = *r_in,
 //      3 with r from the partial sums at r_in;
 // epi: 0 store, 1 add into y, 2 SwiGLU pairs, 3 add into y + rms statistics -> *r_out,
