@@ -1319,17 +1319,34 @@ int q48_gemm_auto_kernel(int T, int N, int K)
     return Q48_GEMM_I8;
 }
 
-int q48_gemm_i8_splits(int T, int N, int K, int cu_count)
+// K splits by an estimate of the time (ns): rounds of blocks over the compute
+// units, each a block's k-steps (0.6 us from planes, 1.3 with the split inside
+// the loop) and its 5 us of prologue and epilogue, then for S > 1 the
+// reduction's launch and its traffic (32 bytes an output and split at about
+// 4.5 TB/s).  Doubling S while the grid was under one block per unit gave two
+// rounds, the second nearly empty, where the tiles divide badly: 128 tokens x
+// 2560 x 2048 took 320 blocks at S = 4, 52.8 us (38.7 prepared), and takes 240 at S
+// = 3, 38.7 us (30.5).
+int q48_gemm_i8_splits(int T, int N, int K, int cu_count, bool planes)
 {
-    const int base = ((N + MN - 1) / MN) * ((T + MT - 1) / MT);
+    const int64_t base = (int64_t)((N + MN - 1) / MN) * ((T + MT - 1) / MT);
     const int steps = (K + MK - 1) / MK;
     const int min_s = (steps + MAXK_RUN / MK - 1) / (MAXK_RUN / MK);
-    int s = 1;
-    // split K while the grid is under one block per compute unit and every
-    // split keeps at least 8 steps
-    while (base * s < cu_count && steps / (2 * s) >= 8)
-        s *= 2;
-    return s > min_s ? s : min_s;
+    const int64_t step = planes ? 600 : 1300;
+    int best = min_s;
+    int64_t cost = INT64_MAX;
+    // 256 x 2048: 16 splits 2-4% faster than 8 to 32 tokens, 2-4% slower from 96
+    const int few = T <= 32 ? 4 : 8;
+    for (int s = min_s; s <= min_s + 63 && (s == min_s || steps / s >= few); ++s) {
+        const int64_t rounds = (base * s + cu_count - 1) / cu_count;
+        const int64_t t = rounds * ((steps + s - 1) / s * step + 5000) +
+                          (s > 1 ? 4500 + 32ll * s * T * N / 4500 : 0);
+        if (t < cost) {
+            cost = t;
+            best = s;
+        }
+    }
+    return best;
 }
 
 size_t q48_gemm_planes_size(int N, int K)
@@ -1354,12 +1371,7 @@ int q48_launch_gemm_prepare(q48_ctx *c, void *Wp, const int64_t *W, int N, int K
 int q48_launch_gemm_i8(q48_ctx *c, int64_t *Y, const int64_t *W, const int64_t *X, int T,
                        int N, int K, int kernel, const void *Wpre)
 {
-    const int S = q48_gemm_i8_splits(T, N, K, c->cu_count);
     const int steps = (K + MK - 1) / MK;
-    const int spb = (steps + S - 1) / S;
-    // blocks (and their redo flags) are numbered in int
-    if ((size_t)((N + MN - 1) / MN) * ((T + MT - 1) / MT) * S > 0x7fffffff)
-        return Q48_EINVAL;
     const int nt = (T + MT - 1) / MT, nn = (N + MN - 1) / MN, nb = nn * nt;
     // the planes path pays one split of X (and of W unless prepared) per
     // call: it wins once tiles are reused enough (measured: T >= 512 with
@@ -1371,6 +1383,11 @@ int q48_launch_gemm_i8(q48_ctx *c, int64_t *Y, const int64_t *W, const int64_t *
         fits && (kernel == Q48_GEMM_I8_PLANES ||
                  (kernel != Q48_GEMM_I8_FUSED && T >= (Wpre ? 2 : 256) && N >= 1024));
     const bool wsplit = planes && !Wpre;
+    const int S = q48_gemm_i8_splits(T, N, K, c->cu_count, planes);
+    const int spb = (steps + S - 1) / S;
+    // blocks (and their redo flags) are numbered in int
+    if ((size_t)((N + MN - 1) / MN) * ((T + MT - 1) / MT) * S > 0x7fffffff)
+        return Q48_EINVAL;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     // workspace: the blocks' redo flags, (S > 1) the int128 partials, then
     // (planes path) X and W digit planes and their masks
