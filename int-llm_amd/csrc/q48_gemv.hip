@@ -290,9 +290,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     // sums of squares (128-bit lo/hi pairs, ceil(K / 8) of them, at most 3
     // per thread); their loads go out first, with the residual's
     // With NTF known each lane preloads np / 64 of the np = K / 8 = 2 NW NTF
-    // partials (16-byte aligned, checked on the host); otherwise they are
-    // read in a loop when needed.
-    constexpr int PC = NTF > 0 ? (NW * SEGC / 8 + 63) / 64 : 1;
+    // partials (16-byte aligned, checked on the host), in the short-row form
+    // its share of those of the longest K; otherwise they are read in a loop
+    // when needed, behind the weights.
+    // Short rows (int64 weights, UNR < 16: every segment at most UNR tiles,
+    // which the host chooses): x is staged in one batch.  The batches of the
+    // general form issue 16 or 32 loads a lane of x and 16 of W whatever K is.
+    constexpr bool SHORT = WT == 0 && NTF == 0 && UNR < 16;
+    constexpr int PC = NTF > 0 ? (NW * SEGC / 8 + 63) / 64 : SHORT ? (2 * NW * UNR + 63) / 64 : 1;
     uint64_t plo[PC], phi[PC];
     const int np = (K + 7) >> 3;
     const uint64_t *st = reinterpret_cast<const uint64_t *>(r_in);
@@ -303,6 +308,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
             const ulonglong2 v = *reinterpret_cast<const ulonglong2 *>(st + 2 * i);
             plo[c] = v.x;
             phi[c] = v.y;
+        }
+    }
+    if (PRO == 3 && SHORT && wave == 0) {
+#pragma unroll
+        for (int c = 0; c < PC; ++c) {
+            const int i = min(lane + c * 64, np - 1);
+            plo[c] = st[2 * i];
+            phi[c] = st[2 * i + 1];
         }
     }
 
@@ -344,7 +357,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     // norm_w are 16-byte aligned (checked on the host): a lane loads element
     // pairs, 16 bytes at a time.  Otherwise single elements, 8 or 16 of them
     // per lane per staging batch.
-    constexpr int XB = NTF > 0 ? (SEGC + 127) / 128 : (PRO ? 8 : 16);
+    constexpr int XB = NTF > 0 ? (SEGC + 127) / 128 : SHORT ? UNR / 4 : (PRO ? 8 : 16);
     constexpr int XW = NTF > 0 ? 2 : 1;   // elements per load
     int64_t xv[XB * XW], nw[XB * XW];
     const int xk = kn > 0 ? k0 : 0, xlast = max(kn - XW, 0);
@@ -396,7 +409,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         // products inside rms_inv_of would contend for the SIMDs
         if (wave == 0) {
             q48_u128 ss = 0;
-            if constexpr (NTF > 0) {
+            if constexpr (NTF > 0 || SHORT) {
 #pragma unroll
                 for (int c = 0; c < PC; ++c) {
                     // masked, not branched: a branch would sink the load and wait
@@ -1260,6 +1273,17 @@ static int launch_v4(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
                            M, K, seg, rkv);
     else if (al && K == NW * seg && seg == 16 * 44)
         hipLaunchKernelGGL((k_gemv_v5<NW, 6, PRO, EPI, 44>), dim3(blocks), dim3(64 * NW), lds,
+                           c->stream, y, W, x, norm_w, r_in, r_out, c->rms_part, c->rms_count,
+                           M, K, seg, rkv);
+    // short rows, K <= 512 and K <= 1024: on the 256-wide model the
+    // normed gate|up took 9.4 us in the general form and takes 5.0, q|k|v 8.8 and
+    // 4.8, W_o 5.5 and 3.5, W_down (K = 688) 5.5 and 4.2
+    else if (seg <= 16 * 4)
+        hipLaunchKernelGGL((k_gemv_v5<NW, 4, PRO, EPI, 0>), dim3(blocks), dim3(64 * NW), lds,
+                           c->stream, y, W, x, norm_w, r_in, r_out, c->rms_part, c->rms_count,
+                           M, K, seg, rkv);
+    else if (seg <= 16 * 8)
+        hipLaunchKernelGGL((k_gemv_v5<NW, 8, PRO, EPI, 0>), dim3(blocks), dim3(64 * NW), lds,
                            c->stream, y, W, x, norm_w, r_in, r_out, c->rms_part, c->rms_count,
                            M, K, seg, rkv);
     else
