@@ -147,6 +147,7 @@ int q48_ctx_create(q48_ctx **out, int device)
     c->attg_wait = q48_attg_default_wait();
     if (hipMalloc(&c->consts, sizeof(q48_consts)) != hipSuccess ||
         hipMalloc(&c->d_scalar, 64 * sizeof(int)) != hipSuccess ||
+        hipHostMalloc((void **)&c->h_token, sizeof(int), hipHostMallocDefault) != hipSuccess ||
         hipMalloc(&c->d_step, 4 * sizeof(int)) != hipSuccess ||
         hipMalloc(&c->amax_part, q48_amax_part_bytes()) != hipSuccess ||
         hipMalloc(&c->rms_count, 512 * sizeof(int)) != hipSuccess ||
@@ -188,6 +189,7 @@ int q48_ctx_destroy(q48_ctx *c)
     (void)hipFree(c->rope_sin);
     (void)hipFree(c->ws);
     (void)hipFree(c->d_scalar);
+    (void)hipHostFree(c->h_token);
     (void)hipFree(c->d_step);
     (void)hipFree(c->amax_part);
     (void)hipFree(c->rms_count);
@@ -561,17 +563,26 @@ int q48_embed(q48_ctx *c, int64_t *out, const int64_t *table, int token, int dim
                                       token, dim));
 }
 
+// The token that the launch just enqueued (its return code rc) writes to the
+// context's word of host memory.  The kernel's own store to mapped host
+// memory replaces a copy of the 4 bytes to pageable memory, which is a launch
+// and a wait of its own: about 20 us of a
+// 256-wide model's 135 a token.
+static int chosen_token(q48_ctx *c, int rc, int *out)
+{
+    if (rc)
+        return rc;
+    if (hipStreamSynchronize(c->stream) != hipSuccess)
+        return Q48_EHIP;
+    *out = *c->h_token;
+    return Q48_OK;
+}
+
 int q48_argmax(q48_ctx *c, const int64_t *v, int n, int *host_out)
 {
     if (!c || !v || !host_out || n <= 0)
         return Q48_EINVAL;
-    int rc = launch_rc(q48_launch_argmax(c, c->d_scalar, v, n));
-    if (rc)
-        return rc;
-    if (hipMemcpyAsync(host_out, c->d_scalar, sizeof(int), hipMemcpyDeviceToHost,
-                       c->stream) != hipSuccess)
-        return Q48_EHIP;
-    return hip_rc(hipStreamSynchronize(c->stream));
+    return chosen_token(c, launch_rc(q48_launch_argmax(c, c->h_token, v, n)), host_out);
 }
 
 int q48_rope_tables(q48_ctx *c, const int64_t **cos_t, const int64_t **sin_t)
@@ -990,7 +1001,7 @@ int q48_embed_stats(q48_ctx *c, int64_t *out, const int64_t *table, int token, i
 // r from the partial sums into the context's scratch word (the fallbacks)
 static int stats_to_r(q48_ctx *c, const int64_t *stats, int dim, int64_t **r)
 {
-    *r = (int64_t *)(c->d_scalar + 16);   // bytes 64..71: clear of the argmax slot
+    *r = (int64_t *)(c->d_scalar + 16);   // bytes 64..71: of the scalar block
     return launch_rc(q48_launch_stats_r(c, *r, stats, dim));
 }
 
@@ -1165,14 +1176,10 @@ int q48_sample(q48_ctx *c, const int64_t *logits, int vocab, int64_t temperature
     int rc = q48_sample_reserve(c, vocab);
     if (rc)
         return rc;
-    rc = launch_rc(q48_launch_sample(c, c->smp, logits, vocab, temperature, top_k, top_p, rng,
-                                     c->d_scalar, nullptr, 0));
-    if (rc)
-        return rc;
-    if (hipMemcpyAsync(token, c->d_scalar, sizeof(int), hipMemcpyDeviceToHost, c->stream) !=
-        hipSuccess)
-        return Q48_EHIP;
-    return hip_rc(hipStreamSynchronize(c->stream));
+    return chosen_token(c,
+                        launch_rc(q48_launch_sample(c, c->smp, logits, vocab, temperature, top_k,
+                                                    top_p, rng, c->h_token, nullptr, 0)),
+                        token);
 }
 
 int q48_sample_step(q48_ctx *c, const int64_t *logits, int vocab, int64_t temperature,

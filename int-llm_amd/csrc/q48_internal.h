@@ -19,7 +19,8 @@ struct q48_ctx {
     int rope_head_dim, rope_max_seq, rope_theta;
     void *ws;                    // device workspace (scores, row sums, partials)
     size_t ws_bytes;
-    int *d_scalar;               // device: small int outputs (argmax)
+    int *d_scalar;               // device: small outputs (norm scalar, bf16_pack's flag)
+    int *h_token;                // host memory that kernels write: a call's chosen token
     int *d_step;                 // device: decode-step state {token, pos, count}
     uint64_t *amax_part;         // device: q48_argmax_step's per-block (max, index) partials,
                                  // then its ticket (back to 0 after use); zeroed at creation

@@ -425,17 +425,46 @@ __device__ __forceinline__ void argmax_scan(const int64_t *__restrict__ v, int n
 #pragma unroll
         for (int b = 0; b < B; ++b) {
             const int i = i0 + tid + 1024 * b;
-            x[b] = v[i < n ? i : n - 1];
+            if (i0 + 1024 * b < n)   // (block-uniform: a short v is a short batch)
+                x[b] = v[i < n ? i : n - 1];
         }
 #pragma unroll
         for (int b = 0; b < B; ++b) {
             const int i = i0 + tid + 1024 * b;
-            if (i < n && x[b] > best) {
+            if (i0 + 1024 * b < n && i < n && x[b] > best) {
                 best = x[b];
                 idx = i;
             }
         }
     }
+}
+
+// The lowest index of the largest value over a block of 1024 threads (n where
+// no thread has one), in every lane of wave 0: per wave the maximum by DPP,
+// then the lowest index among the lanes that hold it, then the same over the
+// 16 waves.  512 values take 5.0 us, its store to host memory included; six
+// shuffle steps of three words, a serial pass over the waves and a scan of 32
+// loads whatever the length took 7.1.
+__device__ __forceinline__ int argmax_block(int64_t best, int idx, int n, int tid,
+                                            int64_t (&bv)[16], int (&bi)[16])
+{
+    const auto wave_first = [&] {
+        const int64_t m = q48_wave_max64(best);
+        idx = -(int)q48_wave_max64(-(int64_t)(best == m ? idx : n));
+        best = m;
+    };
+    wave_first();
+    if ((tid & 63) == 0) {
+        bv[tid >> 6] = best;
+        bi[tid >> 6] = idx;
+    }
+    __syncthreads();
+    if (tid < 64) {
+        best = tid < 16 ? bv[tid] : INT64_MIN;
+        idx = tid < 16 ? bi[tid] : n;
+        wave_first();
+    }
+    return idx;
 }
 
 // ---------------------------------------------------------------------------
@@ -1366,26 +1395,8 @@ __global__ __launch_bounds__(1024) void k_step_argmax(int *__restrict__ st,
     int64_t best = INT64_MIN;
     int idx = n;
     argmax_scan(v, n, tid, best, idx);
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const int64_t ov = __shfl_xor(best, off, 64);
-        const int oi = __shfl_xor(idx, off, 64);
-        if (ov > best || (ov == best && oi < idx)) {
-            best = ov;
-            idx = oi;
-        }
-    }
-    if ((tid & 63) == 0) {
-        bv[tid >> 6] = best;
-        bi[tid >> 6] = idx;
-    }
-    __syncthreads();
+    idx = argmax_block(best, idx, n, tid, bv, bi);
     if (tid == 0) {
-        for (int w = 1; w < 16; ++w)
-            if (bv[w] > best || (bv[w] == best && bi[w] < idx)) {
-                best = bv[w];
-                idx = bi[w];
-            }
         const int tok = idx < n ? idx : 0;
         st[0] = tok;
         st[1] = st[1] + 1;
@@ -1465,26 +1476,8 @@ __global__ __launch_bounds__(1024) void k_argmax(int *__restrict__ out,
     int64_t best = INT64_MIN;
     int idx = n;   // sentinel larger than any index
     argmax_scan(v, n, tid, best, idx);
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const int64_t ov = __shfl_xor(best, off, 64);
-        const int oi = __shfl_xor(idx, off, 64);
-        if (ov > best || (ov == best && oi < idx)) {
-            best = ov;
-            idx = oi;
-        }
-    }
-    if ((tid & 63) == 0) {
-        bv[tid >> 6] = best;
-        bi[tid >> 6] = idx;
-    }
-    __syncthreads();
+    idx = argmax_block(best, idx, n, tid, bv, bi);
     if (tid == 0) {
-        for (int w = 1; w < 16; ++w)
-            if (bv[w] > best || (bv[w] == best && bi[w] < idx)) {
-                best = bv[w];
-                idx = bi[w];
-            }
         *out = idx < n ? idx : 0;
     }
 }

@@ -1,6 +1,6 @@
 """The fused GEMVs on short rows (int64 weights, K <= 512 and K <= 1024 staged
 in one batch): lengths about the tiles, the segments and both limits, against
-the oracle."""
+the oracle; and the block argmax's ties and extremes."""
 import numpy as np
 import pytest
 
@@ -62,3 +62,16 @@ def test_short_rows_vs_oracle(ctx, oracle, K):
         assert int(words[2 * b]) + (int(words[2 * b + 1]) << 64) == ss, b
     for b in (dW, dx, dw, ds, dt, dy, do, dh, dxf):
         b.free()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 1024, 1025, 32767, 32769])
+def test_argmax_first_of_equals(ctx, n):
+    rng = np.random.default_rng(n)
+    for v in (np.full(n, spec.INT64_MIN, dtype=np.int64),
+              np.full(n, spec.INT64_MAX, dtype=np.int64),
+              rng.integers(-2, 2, size=n, dtype=np.int64),
+              np.arange(n, dtype=np.int64), -np.arange(n, dtype=np.int64)):
+        dv = ctx.to_device(v)
+        print("[case] argmax", n, flush=True)
+        assert ctx.argmax(dv.ptr, n) == int(np.argmax(v))
+        dv.free()
