@@ -882,7 +882,7 @@ __device__ __forceinline__ void mfma_i8(v16i (&acc)[NW][11], int n, int r, const
         mfma_asm<false>(acc[n][r], a, b);
 }
 // The sums after the k loop: an MFMA's result may be read by other vector
-// instructions only after its passes (at most 18 wait states), which the
+// instructions only after its passes (at most 20 wait states), which the
 // compiler adds before the instructions it knows but not around mfma_asm and
 // mad_shl_asm; what reads a sum depends on this.
 template <int NW>
@@ -1111,6 +1111,14 @@ __device__ __forceinline__ void planes_pass(uint8_t (&s0)[stage_bytes(NW)],
         e1 = e5;
         e2 = e6;
         e3 = e7;
+        // mfma_asm's wait states, here too: copies of the sums that the register
+        // allocator puts between the loop and mfma_settle read them (16 passes
+        // need 20; the next group's first wait and barrier follow anyway)
+        if constexpr (NW > 1) {
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_nop 15\n\ts_nop 3");
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     wait_vm<0>();   // no DMA in flight when the block gives its LDS back
 }
