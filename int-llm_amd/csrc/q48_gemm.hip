@@ -1391,8 +1391,15 @@ int q48_launch_gemm_i8(q48_ctx *c, int64_t *Y, const int64_t *W, const int64_t *
         fits && (kernel == Q48_GEMM_I8_PLANES ||
                  (kernel != Q48_GEMM_I8_FUSED && T >= (Wpre ? 2 : 256) && N >= 1024));
     const bool wsplit = planes && !Wpre;
-    const int S = q48_gemm_i8_splits(T, N, K, c->cu_count, planes);
-    const int spb = (steps + S - 1) / S;
+    int S = q48_gemm_i8_splits(T, N, K, c->cu_count, planes);
+    int spb = (steps + S - 1) / S;
+    // planes_pass reaches a row tile's zero X planes by a 32-bit offset from
+    // the split's start.  Where that can pass 4 GB only the last split, which
+    // they follow directly, may need them: whole groups of four steps elsewhere
+    if (planes && (size_t)steps * 8 * PLANE > 0xffffffffu) {
+        spb = min((spb + 3) & ~3, MAXK_RUN / MK & ~3);
+        S = (steps + spb - 1) / spb;
+    }
     // blocks (and their redo flags) are numbered in int
     if ((size_t)((N + MN - 1) / MN) * ((T + MT - 1) / MT) * S > 0x7fffffff)
         return Q48_EINVAL;

@@ -87,3 +87,27 @@ def test_block_numbering():
     for nn in range(1, 30):
         for nt in range(1, 12):
             assert all(block_of(*tile_of(b, nn, nt), nn, nt) == b for b in range(nn * nt))
+
+
+@pytest.mark.gpu
+def test_gemm_long_k_vs_oracle(oracle):
+    """A row tile of more than 4 GB of digit planes: its zero planes, which fill
+    up a split's last group of four k-steps, are past a 32-bit offset from the
+    first splits, whose lengths are therefore multiples of four."""
+    import intllm
+    T, N, K = 2, 3, 32 * (262144 + 601) - 5
+    rng = np.random.default_rng(11)
+    W = np.ascontiguousarray(weights("bf16", rng, N, K)).ravel()
+    X = (rng.standard_normal(T * K) * ONE).astype(np.int64)
+    want = np.empty(T * N, dtype=np.int64)
+    oracle.q48o_gemm(want.ctypes.data, W.ctypes.data, X.ctypes.data, T, N, K)
+    ctx = intllm.Context(0)   # its own: 9 GB of workspace go with it
+    dW, dX, dY = ctx.to_device(W), ctx.to_device(X), ctx.buffer(T * N)
+    try:
+        print("[case] gemm long k", T, N, K, flush=True)
+        ctx.gemm(dY.ptr, dW.ptr, dX.ptr, T, N, K, intllm.GEMM_I8_PLANES)
+        assert np.array_equal(dY.download(), want)
+    finally:
+        for b in (dW, dX, dY):
+            b.free()
+        ctx.close()
