@@ -663,16 +663,31 @@ __global__ __launch_bounds__(256) void k_gemm_i8_reduce(int64_t *__restrict__ Y,
 // ---------------------------------------------------------------------------
 
 // The shift of each 64-row tile's planes (k_planes) from its largest
-// magnitude, left in bits 16..18 of the row tile's first mask word: one block
-// per row tile.
+// magnitude.  Block (rt, p) of grid (nn, parts) takes the p-th of the row
+// tile's parts and leaves its magnitude's code in bits 20..25 of the row
+// tile's p-th mask word: 8 h + 7 - shift, h the plane its largest magnitude
+// fills, which grows with the magnitude, so k_planes takes the parts' largest.
+// Parts of about 8192 values, one load batch a thread, fill the chip at any
+// size: with a block per row tile the pass was a chain of K / 128 batches on
+// N / 64 compute units (q48_gemm_prepare of 1024 x 1024 10.3 -> 7.3 us, 2048 x
+// 2048 23.4 -> 18.3, 2048 x 5632 55.6 -> 40.3; 11264 x 2048 88.4 -> 87.4).
+constexpr int TS_PARTS = 16;
+__host__ __device__ __forceinline__ int tile_parts(int K, int nsteps)
+{
+    const int p = (K + 127) / 128;
+    return min(min(p, nsteps), TS_PARTS);
+}
 __global__ __launch_bounds__(1024) void k_tile_shift(uint32_t *__restrict__ mask,
                                                     const int64_t *__restrict__ src, int R,
                                                     int K, int nsteps)
 {
     __shared__ uint64_t red[16];
     const int tid = threadIdx.x, r0 = (int)blockIdx.x * MN, r1 = min(r0 + MN, R);
-    const int64_t *p = src + (size_t)r0 * K;
-    const size_t n = (size_t)(r1 - r0) * K;
+    const size_t all = (size_t)(r1 - r0) * K;
+    // whole 8192s a part, the last takes what is left (possibly nothing)
+    const size_t per = ((all + gridDim.y - 1) / gridDim.y + 8191) & ~(size_t)8191;
+    const size_t b = min(all, per * blockIdx.y), n = min(all - b, per);
+    const int64_t *p = src + (size_t)r0 * K + b;
     uint64_t mx = 0;
     auto add = [&](uint64_t v) {
         const uint64_t a = (int64_t)v < 0 ? (uint64_t)0 - v : v;
@@ -708,12 +723,14 @@ __global__ __launch_bounds__(1024) void k_tile_shift(uint32_t *__restrict__ mask
         // the lowest plane h <= 6 whose digits reach mx (values up to
         // sum_{i<=h} 127 256^i), and the largest shift that stays within it
         uint64_t lim = 127;
-        for (int h = 0; h < 6 && mx > lim; ++h)
+        uint32_t h = 0;
+        for (; h < 6 && mx > lim; ++h)
             lim = lim * 256 + 127;
         uint32_t sh = 0;
         while (sh < 7 && (mx << (sh + 1)) <= lim)
             ++sh;
-        mask[(size_t)blockIdx.x * nsteps] = mx <= lim ? sh << 16 : 0;
+        mask[(size_t)blockIdx.x * nsteps + blockIdx.y] =
+            (mx <= lim ? 8 * h + 7 - sh : 63u) << 20;
     }
 }
 
@@ -727,9 +744,9 @@ __global__ __launch_bounds__(1024) void k_tile_shift(uint32_t *__restrict__ mask
 // pitch: blocks per row tile, one past nsteps holding zero planes (X: nsteps + 1,
 // for the steps that fill up the k loop's groups of four; W: nsteps).
 // shifted: the row tile's values are multiplied by 2^shift before the split
-// (bits 16..18 of its first mask word, from k_tile_shift; every mask of the
-// row tile keeps them, so a block may read them before or after the first
-// block writes its own mask), so that the largest one fills its top plane: a
+// (from the largest code of k_tile_shift's parts; every mask of the row tile
+// keeps that code, so a block may read a part's word before or after the
+// block that writes its own mask there; bits 16..18: the shift), so that the largest one fills its top plane: a
 // bfloat16 weight's low bits then reach down to fewer planes (N(0, 0.02)
 // weights: 10% of the 64 x 32 tiles need a fourth plane, 34% unshifted).
 __global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst, uint32_t *mask,
@@ -762,10 +779,14 @@ __global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst, uint3
         for (int e = 0; e < 8; ++e)
             v[e] = row < R && k0 + e < K ? (uint64_t)rp[e] : 0;
     }
-    const uint32_t sh =
-        shifted ? (__hip_atomic_load(mask + (size_t)rt * nsteps, __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT) >> 16) & 7u
-                : 0u;
+    uint32_t sh = 0, code = 0;
+    if (shifted) {
+        const int part = min(tid & (TS_PARTS - 1), tile_parts(K, nsteps) - 1);
+        code = (__hip_atomic_load(mask + (size_t)rt * nsteps + part, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT) >> 20) & 63u;
+        code = (uint32_t)q48_wave_max64((int64_t)code);
+        sh = 7u - (code & 7u);
+    }
     if (sh)
 #pragma unroll
         for (int e = 0; e < 8; ++e)
@@ -793,7 +814,7 @@ __global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst, uint3
         d[4 + a] = make_uint2(h0[a] ^ 0x80808080u, h1[a] ^ 0x80808080u);
     d[7] = make_uint2(h0[3], h1[3]);
     uint8_t *p = dst + (size_t)blockIdx.x * 8 * PLANE + pc.off;
-    uint32_t m = (big ? 0x100u : 0u) | (sh << 16);
+    uint32_t m = (big ? 0x100u : 0u) | (sh << 16) | (code << 20);
 #pragma unroll
     for (int a = 0; a < 8; ++a) {
         *reinterpret_cast<uint2 *>(p + a * PLANE) = d[a];
@@ -1370,7 +1391,8 @@ int q48_launch_gemm_prepare(q48_ctx *c, void *Wp, const int64_t *W, int N, int K
         return Q48_EINVAL;
     uint8_t *p = (uint8_t *)Wp;
     uint32_t *m = (uint32_t *)(p + (size_t)nn * steps * 8 * PLANE);
-    hipLaunchKernelGGL(k_tile_shift, dim3(nn), dim3(1024), 0, c->stream, m, W, N, K, steps);
+    hipLaunchKernelGGL(k_tile_shift, dim3(nn, tile_parts(K, steps)), dim3(1024), 0, c->stream, m,
+                       W, N, K, steps);
     hipLaunchKernelGGL(k_planes, dim3(nn * steps), dim3(256), 0, c->stream, p, m, W, N, K,
                        steps, steps, 1);
     return (int)hipGetLastError();
