@@ -70,13 +70,29 @@ __device__ __forceinline__ int64_t q48_mul_shr(int64_t a, int64_t b)
 // nearest needs five dependent operations for the same value (product,
 // floor, remainder, floor, add).  Called at the top of every kernel that
 // uses q48_inv_sqrt, q48_exp_small (q48_safe_exp, q48_sigmoid, q48_silu),
-// q48_recip or q48_divisor_of / q48_div_by, which are written for this mode;
-// the general divisions (q48_div, q48_divs_128_64) are exact in either: their
-// estimates are corrected by integer remainders.  The clobber keeps loads,
-// and so the arithmetic on what they load, below the switch.
+// q48_exp_neg, q48_recip, q48_divisor_of / q48_div_by or the FP64 sums, which
+// are written for this mode; the general divisions (q48_div, q48_divs_128_64)
+// are exact in either: their estimates are corrected by integer remainders.
+//
+// The compiler does not know that FP64 arithmetic depends on the mode, so the
+// order is not its promise.  What keeps the arithmetic below the switch: it
+// works on loaded values, and the memory clobber keeps loads that are not of
+// const __restrict__ data below; a value that comes from kernel arguments or
+// such loads goes through q48_below where the arithmetic on it is all there
+// is.  tests/test_device_code.py checks every kernel of the built library:
+// the switch before the first branch and before the first FP64 operation.
+// (__builtin_amdgcn_s_setreg is no way out: the compiler then knows that the
+// mode has changed, and sets it back to nearest before FP64 arithmetic.)
 __device__ __forceinline__ void q48_round_down()
 {
     asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 2" ::: "memory");
+}
+
+// v, as a value that exists only below the asm statements above it
+__device__ __forceinline__ int64_t q48_below(int64_t v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
 }
 
 // The integer v of a double v + 2^52 (0 <= v < 2^52), from its word; as a

@@ -71,6 +71,7 @@ __global__ __launch_bounds__(256) void k_rope_init(int64_t *__restrict__ cos_t,
                                                   const q48_consts *__restrict__ k,
                                                   int head_dim, int max_seq, int theta)
 {
+    q48_round_down();
     const int half = head_dim / 2;
     const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (long)half * max_seq)
@@ -83,10 +84,8 @@ __global__ __launch_bounds__(256) void k_rope_init(int64_t *__restrict__ cos_t,
     q48_sincos(k, q48_mul(q48_from_int(pos), th), &c, &s);
     cos_t[idx] = c;
     sin_t[idx] = s;
-    if (idx == 0) {   // the attention score scale, stored after the sine table
-        q48_round_down();
-        sin_t[(size_t)half * max_seq] = q48_inv_sqrt(q48_from_int(head_dim));
-    }
+    if (idx == 0)   // the attention score scale, stored after the sine table
+        sin_t[(size_t)half * max_seq] = q48_inv_sqrt(q48_below(q48_from_int(head_dim)));
 }
 
 // ---------------------------------------------------------------------------
@@ -1496,36 +1495,47 @@ __global__ void k_zero_bytes(uint8_t *__restrict__ p, size_t n)
         p[i] = 0;
 }
 
-// Element-wise fp_math evaluation (determinism gate and unit parity).
+// Element-wise fp_math evaluation (determinism gate and unit parity).  DOWN:
+// the functions written for FP64 rounding down (q48_round_down), which the
+// others are evaluated without.
+static bool fp_eval_down(int func)
+{
+    return func == 4 || (func >= 8 && func <= 10) || func == 12;
+}
+template <bool DOWN>
 __global__ __launch_bounds__(256) void k_fp_eval(int func, const int64_t *__restrict__ x,
                                                 const int64_t *__restrict__ y,
                                                 int64_t *__restrict__ o0,
                                                 int64_t *__restrict__ o1,
                                                 const q48_consts *__restrict__ k, int n)
 {
+    if constexpr (DOWN)
+        q48_round_down();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n)
         return;
-    // the functions written for rounding down; the others keep the default
-    if (func == 4 || (func >= 8 && func <= 10) || func == 12)
-        q48_round_down();
-    const int64_t a = x[i];
+    const int64_t a = q48_below(x[i]);
     int64_t r = 0, r1 = 0;
-    switch (func) {
-    case 0: r = q48_mul(a, y[i]); break;
-    case 1: r = y[i] != 0 ? q48_div(a, y[i]) : 0; break;
-    case 2: r = q48_sqrt(a); break;
-    case 3: r = q48_sqrt_fast(a); break;
-    case 4: r = q48_inv_sqrt(a); break;
-    case 5: r = q48_exp(a); break;
-    case 6: r = q48_log(a); break;
-    case 7: q48_sincos(k, a, &r, &r1); break;
-    case 8: r = q48_sigmoid(a); break;
-    case 9: r = q48_silu(a); break;
-    case 10: r = q48_safe_exp(a); break;
-    case 11: r = q48_exp_dyadic(a, (int)y[i]); break;
-    case 12: r = y[i] != 0 ? q48_div_by(a, q48_divisor_of(y[i])) : 0; break;
-    default: break;
+    if constexpr (DOWN) {
+        switch (func) {
+        case 4: r = q48_inv_sqrt(a); break;
+        case 8: r = q48_sigmoid(a); break;
+        case 9: r = q48_silu(a); break;
+        case 10: r = q48_safe_exp(a); break;
+        default: r = y[i] != 0 ? q48_div_by(a, q48_divisor_of(q48_below(y[i]))) : 0; break;
+        }
+    } else {
+        switch (func) {
+        case 0: r = q48_mul(a, y[i]); break;
+        case 1: r = y[i] != 0 ? q48_div(a, y[i]) : 0; break;
+        case 2: r = q48_sqrt(a); break;
+        case 3: r = q48_sqrt_fast(a); break;
+        case 5: r = q48_exp(a); break;
+        case 6: r = q48_log(a); break;
+        case 7: q48_sincos(k, a, &r, &r1); break;
+        case 11: r = q48_exp_dyadic(a, (int)y[i]); break;
+        default: break;
+        }
     }
     o0[i] = r;
     if (o1)
@@ -1888,7 +1898,8 @@ int q48_launch_zero(q48_ctx *c, void *p, size_t bytes)
 int q48_launch_fp_eval(q48_ctx *c, int func, const int64_t *x,
                        const int64_t *y, int64_t *out0, int64_t *out1, int n)
 {
-    hipLaunchKernelGGL(k_fp_eval, dim3((n + 255) / 256), dim3(256), 0, c->stream, func, x, y,
-                       out0, out1, c->consts, n);
+    hipLaunchKernelGGL(fp_eval_down(func) ? k_fp_eval<true> : k_fp_eval<false>,
+                       dim3((n + 255) / 256), dim3(256), 0, c->stream, func, x, y, out0, out1,
+                       c->consts, n);
     return (int)hipGetLastError();
 }
