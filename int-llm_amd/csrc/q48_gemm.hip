@@ -902,10 +902,27 @@ __device__ __forceinline__ void mfma_i8(v16i (&acc)[NW][11], int n, int r, const
     else
         mfma_asm<false>(acc[n][r], a, b);
 }
-// The sums after the k loop: an MFMA's result may be read by other vector
-// instructions only after its passes (at most 20 wait states), which the
-// compiler adds before the instructions it knows but not around mfma_asm and
-// mad_shl_asm; what reads a sum depends on this.
+// An MFMA's result may be touched by other vector instructions only after its
+// passes: 12 wait states here, which the compiler keeps itself after the
+// instructions it knows, but not after mfma_asm.  Nothing in the source touches
+// a sum between the MFMAs, but the register allocator may put copies of sums
+// at the joins of the control flow; so the waits end every path that leaves
+// mfma_asm behind: the conditional MFMAs of a step, each group of four steps,
+// and the loop (mfma_settle).  Inside a group the steps follow each other
+// without one (12 states are about 50 cycles, the step's 42 MFMAs 1350): that no
+// path of the built code touches a sum too early is checked there, by
+// tests/test_device_code.py.
+template <int NW>
+__device__ __forceinline__ void mfma_wait()
+{
+    if constexpr (NW > 1) {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_nop 11");
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+// The sums after the k loop, what reads them depending on this (mad_shl_asm is
+// as unknown to the compiler as mfma_asm).
 template <int NW>
 __device__ __forceinline__ void mfma_settle(v16i (&acc)[NW][11])
 {
@@ -1053,6 +1070,7 @@ __device__ __forceinline__ void planes_pass(uint8_t (&s0)[stage_bytes(NW)],
                     for (int a = 0; a < 7; ++a)
                         mfma_i8(acc, n, a, o.A[a], Bx);
                 }
+            mfma_wait<NW>();
         }
         v4i nb[NW][3], a6;
         __builtin_amdgcn_sched_barrier(0);
@@ -1132,14 +1150,7 @@ __device__ __forceinline__ void planes_pass(uint8_t (&s0)[stage_bytes(NW)],
         e1 = e5;
         e2 = e6;
         e3 = e7;
-        // mfma_asm's wait states, here too: copies of the sums that the register
-        // allocator puts between the loop and mfma_settle read them (16 passes
-        // need 20; the next group's first wait and barrier follow anyway)
-        if constexpr (NW > 1) {
-            __builtin_amdgcn_sched_barrier(0);
-            asm volatile("s_nop 15\n\ts_nop 3");
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        mfma_wait<NW>();   // the next group's first wait and barrier follow anyway
     }
     wait_vm<0>();   // no DMA in flight when the block gives its LDS back
 }
