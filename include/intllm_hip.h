@@ -169,7 +169,9 @@ int q48_fp_eval(q48_ctx *ctx, int func, const int64_t *x, const int64_t *y,
 
 /* ---- fused decode ops ------------------------------------------------------- */
 /* Each is exactly the composition it names (same bits as the separate ops);
- * fusing removes launches and a round trip of the activation through HBM. */
+ * fusing removes launches and a round trip of the activation through HBM.
+ * With int64 weights an output may share words with the vectors a GEMV reads
+ * (not with W): such a call runs as separate launches through a temporary. */
 
 /* y = W . rmsnorm(x, norm_w): rmsnorm (llama_int.c:1048-1058) followed by
  * matmul_vec (llama_int.c:1014-1046), K = dim of x.  Used for q|k|v

@@ -6,6 +6,7 @@
 #include "../../include/intllm_hip.h"
 #include "q48_internal.h"
 
+#include <initializer_list>
 #include <new>
 #include <stdlib.h>
 
@@ -635,6 +636,37 @@ bool bad_ptrs(const void *a, const void *b, const void *d)
 {
     return !a || !b || !d || ((((uintptr_t)a) | ((uintptr_t)b) | ((uintptr_t)d)) & 7);
 }
+
+// Words of a vector operand, and whether an output shares some with it.
+struct Words {
+    const int64_t *p;
+    size_t n;
+};
+bool meets(Words a, Words b)
+{
+    return a.p && b.p && (uintptr_t)a.p < (uintptr_t)(b.p + b.n) &&
+           (uintptr_t)b.p < (uintptr_t)(a.p + a.n);
+}
+
+// Whether a GEMV and what surrounds it may be one launch.  Its blocks write
+// their rows while others still read the vectors, so an output that shares
+// words with one of them takes the separate launches, which go through a
+// temporary.  (A single block reads all it needs before it writes; with even K
+// and aligned W such a call stays one launch, which needs no temporary, as a
+// capture may demand.)
+bool one_launch(const int64_t *W, int M, int K, std::initializer_list<Words> out,
+                std::initializer_list<Words> in)
+{
+    if (!q48_gemv_v5_ok(M, K))
+        return false;
+    if (M <= 8 && q48_gemv_v2_ok(W, K))
+        return true;
+    for (const Words &o : out)
+        for (const Words &i : in)
+            if (meets(o, i))
+                return false;
+    return true;
+}
 } // namespace
 
 int q48_rmsnorm_gemv(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
@@ -642,7 +674,7 @@ int q48_rmsnorm_gemv(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
 {
     if (!c || bad_ptrs(y, W, x) || !norm_w || M <= 0 || K <= 0 || M > kMaxDim || K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v5_ok(M, K)) {
+    if (one_launch(W, M, K, {{y, (size_t)M}}, {{x, (size_t)K}, {norm_w, (size_t)K}})) {
         int prc;
         q48_ctx::ProfRec *r = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -662,7 +694,7 @@ int q48_gemv_residual(q48_ctx *c, int64_t *acc, const int64_t *W, const int64_t 
 {
     if (!c || bad_ptrs(acc, W, x) || M <= 0 || K <= 0 || M > kMaxDim || K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v5_ok(M, K)) {
+    if (one_launch(W, M, K, {{acc, (size_t)M}}, {{x, (size_t)K}})) {
         int prc;
         q48_ctx::ProfRec *r = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -683,7 +715,8 @@ int q48_rmsnorm_gemv_swiglu(q48_ctx *c, int64_t *out, const int64_t *Wgu, const 
     if (!c || bad_ptrs(out, Wgu, x) || !norm_w || ffn <= 0 || K <= 0 || ffn > kMaxDim / 2 ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v5_ok(2 * ffn, K)) {
+    if (one_launch(Wgu, 2 * ffn, K, {{out, (size_t)ffn}},
+                   {{x, (size_t)K}, {norm_w, (size_t)K}})) {
         int prc;
         q48_ctx::ProfRec *r = prof_begin(c, gemv_bytes(2 * ffn, K, ffn), &prc);
         if (prc)
@@ -914,7 +947,7 @@ int q48_norm_gemv(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
     if (!c || bad_ptrs(y, W, x) || !norm_w || !r || M <= 0 || K <= 0 || M > kMaxDim ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v5_ok(M, K)) {
+    if (one_launch(W, M, K, {{y, (size_t)M}}, {{x, (size_t)K}, {norm_w, (size_t)K}, {r, 1}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -936,7 +969,8 @@ int q48_norm_gemv_swiglu(q48_ctx *c, int64_t *out, const int64_t *Wgu, const int
     if (!c || bad_ptrs(out, Wgu, x) || !norm_w || !r || ffn <= 0 || K <= 0 ||
         ffn > kMaxDim / 2 || K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v5_ok(2 * ffn, K)) {
+    if (one_launch(Wgu, 2 * ffn, K, {{out, (size_t)ffn}},
+                   {{x, (size_t)K}, {norm_w, (size_t)K}, {r, 1}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(2 * ffn, K, ffn), &prc);
         if (prc)
@@ -960,7 +994,7 @@ int q48_gemv_residual_rms(q48_ctx *c, int64_t *acc, const int64_t *W, const int6
     if (!c || bad_ptrs(acc, W, x) || !r_out || M <= 0 || K <= 0 || M > kMaxDim ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v5_ok(M, K)) {
+    if (one_launch(W, M, K, {{acc, (size_t)M}, {r_out, 1}}, {{x, (size_t)K}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -1011,7 +1045,8 @@ int q48_norm_gemv_stats(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t 
     if (!c || bad_ptrs(y, W, x) || !norm_w || !stats || M <= 0 || K <= 0 || M > kMaxDim ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v5_ok(M, K)) {
+    if (one_launch(W, M, K, {{y, (size_t)M}},
+                   {{x, (size_t)K}, {norm_w, (size_t)K}, {stats, (size_t)Q48_STATS_WORDS(K)}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -1030,7 +1065,8 @@ int q48_norm_gemv_swiglu_stats(q48_ctx *c, int64_t *out, const int64_t *Wgu, con
     if (!c || bad_ptrs(out, Wgu, x) || !norm_w || !stats || ffn <= 0 || K <= 0 ||
         ffn > kMaxDim / 2 || K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v5_ok(2 * ffn, K)) {
+    if (one_launch(Wgu, 2 * ffn, K, {{out, (size_t)ffn}},
+                   {{x, (size_t)K}, {norm_w, (size_t)K}, {stats, (size_t)Q48_STATS_WORDS(K)}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(2 * ffn, K, ffn), &prc);
         if (prc)
@@ -1048,7 +1084,8 @@ int q48_gemv_residual_stats(q48_ctx *c, int64_t *acc, const int64_t *W, const in
 {
     if (!c || bad_ptrs(acc, W, x) || !stats || M <= 0 || K <= 0 || M > kMaxDim || K > kMaxDim)
         return Q48_EINVAL;
-    if (q48_gemv_v5_ok(M, K)) {
+    if (one_launch(W, M, K, {{acc, (size_t)M}, {stats, (size_t)Q48_STATS_WORDS(M)}},
+                   {{x, (size_t)K}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)

@@ -1623,9 +1623,12 @@ int q48_launch_gemv(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
     if ((K == 2048 || K == 5632) && (((uintptr_t)W | (uintptr_t)x) & 15) == 0)
         return launch_v4<0, 0>(c, y, W, x, nullptr, nullptr, nullptr, M, K);
     // waves per row: until 2048 waves (8 a compute unit) or one tile each;
-    // many short rows: four a wave, for the loads in flight and x read once
+    // many short rows: four a wave, for the loads in flight and x read once.
+    // y over x (8 rows at most, one block): one wave a row, which reads all of
+    // x before the block stores
     int S = 1;
-    while (S < 8 && (size_t)M * S < 2048 && K / (2 * S) >= 128)
+    const bool over = M <= 8 && (uintptr_t)y < (uintptr_t)(x + K) && (uintptr_t)x < (uintptr_t)(y + M);
+    while (!over && S < 8 && (size_t)M * S < 2048 && K / (2 * S) >= 128)
         S *= 2;
     const int seg = S == 1 ? K : ((K + S - 1) / S + 1) & ~1;
     auto go = [&](auto kern, int rows) {
