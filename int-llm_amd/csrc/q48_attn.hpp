@@ -87,11 +87,9 @@ __device__ __forceinline__ void attn_v3_head(
     __shared__ int64_t red[NT / 64], red2[NT / 64];
     __shared__ int64_t part[NT];
     __shared__ int64_t sc[SMAX];
-    __shared__ int form, big_v;   // set by any thread that sees the case, below
-    if (threadIdx.x == 0) {
+    __shared__ int form;   // of the weights, set by any thread that sees the case, below
+    if (threadIdx.x == 0)
         form = 0;
-        big_v = 0;
-    }
     if (!ROT) {
         if (d_pos)
             pos = *d_pos;
@@ -279,27 +277,44 @@ __device__ __forceinline__ void attn_v3_head(
     // lane l of a row of 16 holds the weight of its slice's position i0 + l
     // % 16 (0 past S).  17 VALU operations and an LDS read per term became
     // about five operations and no read: 9.5 -> 8.5 us a call at 121 positions.
+    // A batch of values is tested before its terms are added: at the first one
+    // out of q48_f51's range the wave goes on with the general products, from
+    // that batch on (half2: the second of the pair at i0).  With such a value
+    // in each head a call takes 9.5 us at 121 positions and 13.4 at 251; a pass
+    // to the end, tested there and then redone, took 11.1 and 17.0, the general
+    // products alone 9.6 and 14.3.
     double facc = Q48_FSUM0;
-    uint32_t big = 0;
+    int i0 = 0;
+    bool half2 = false;
     if (!wide) {
-        auto fmac = [&](auto base, const int64_t(&vv)[VB], int i0, double p) {
+        // true: every lane's values are in range, and their terms are added
+        auto fmac = [&](auto base, const int64_t(&vv)[VB], double p) -> bool {
             double f[VB];
+            uint32_t big = 0;
 #pragma unroll
             for (int u = 0; u < VB; ++u)
-                f[u] = q48_f51(!ROT && sl + SL * (i0 + u) == pos ? vs[d] : vv[u], big);
+                f[u] = q48_f51(!ROT && sl + SL * (i0 + decltype(base)::value + u) == pos ? vs[d]
+                                                                                         : vv[u],
+                               big);
+            if (__ballot(q48_f51_big(big)))
+                return false;
             q48_fsum8<decltype(base)::value>(facc, p, f);
+            return true;
         };
-        for (int i0 = 0; sl + SL * i0 < S; i0 += 2 * VB) {
+        for (; sl + SL * i0 < S; i0 += 2 * VB) {
             const int tp = sl + SL * (i0 + (tid & 15));
             const double p = tp < S ? q48_pscaled(sc[tp]) : 0.0;
-            fmac(std::integral_constant<int, 0>{}, va, i0, p);
+            if (!fmac(std::integral_constant<int, 0>{}, va, p))
+                break;
             if (SL * (i0 + 2 * VB) < S) {
 #pragma unroll
                 for (int u = 0; u < VB; ++u)
                     va[u] = vld(i0 + 2 * VB + u);
             }
-            if (SL * (i0 + VB) < S)
-                fmac(std::integral_constant<int, VB>{}, vb, i0 + VB, p);
+            if (SL * (i0 + VB) < S && !fmac(std::integral_constant<int, VB>{}, vb, p)) {
+                half2 = true;
+                break;
+            }
             if (SL * (i0 + 3 * VB) < S) {
 #pragma unroll
                 for (int u = 0; u < VB; ++u)
@@ -307,21 +322,15 @@ __device__ __forceinline__ void attn_v3_head(
             }
         }
     }
-    part[tid] = q48_fsum_total(facc);
-    if (q48_f51_big(big))
-        big_v = 1;
-    __syncthreads();
-    const bool over = wide || big_v;
 
-    // the general products, where a weight or a value is out of that range;
-    // one copy of the loop per product form
+    // the general products of what is left, one copy of the loop per product form
     auto values = [&](auto nonneg) -> uint64_t {
         uint64_t acc = 0;
         q48_pv_acc pa = {0, 0};
-        auto vmac = [&](const int64_t(&vv)[VB], int i0) {
+        auto vmac = [&](const int64_t(&vv)[VB], int j0) {
 #pragma unroll
             for (int u = 0; u < VB; ++u) {
-                const int t = sl + SL * (i0 + u);
+                const int t = sl + SL * (j0 + u);
                 if (t < S) {
                     const int64_t v = !ROT && t == pos ? vs[d] : vv[u];
                     if constexpr (decltype(nonneg)::value)
@@ -331,20 +340,17 @@ __device__ __forceinline__ void attn_v3_head(
                 }
             }
         };
-#pragma unroll
-        for (int u = 0; u < VB; ++u)
-            va[u] = vld(u);
-#pragma unroll
-        for (int u = 0; u < VB; ++u)
-            vb[u] = vld(VB + u);
-        for (int i0 = 0; sl + SL * i0 < S; i0 += 2 * VB) {
+        for (; sl + SL * i0 < S; i0 += 2 * VB) {
             // the next batches where some position of them exists (as above)
-            vmac(va, i0);
-            if (SL * (i0 + 2 * VB) < S) {
+            if (!half2) {
+                vmac(va, i0);
+                if (SL * (i0 + 2 * VB) < S) {
 #pragma unroll
-                for (int u = 0; u < VB; ++u)
-                    va[u] = vld(i0 + 2 * VB + u);
+                    for (int u = 0; u < VB; ++u)
+                        va[u] = vld(i0 + 2 * VB + u);
+                }
             }
+            half2 = false;
             if (SL * (i0 + VB) < S)
                 vmac(vb, i0 + VB);
             if (SL * (i0 + 3 * VB) < S) {
@@ -355,10 +361,9 @@ __device__ __forceinline__ void attn_v3_head(
         }
         return acc + (uint64_t)q48_pv_total(pa);
     };
-    if (over) {   // uniform over the block
-        part[tid] = (int64_t)(neg ? values(std::false_type{}) : values(std::true_type{}));
-        __syncthreads();
-    }
+    part[tid] = (int64_t)((uint64_t)q48_fsum_total(facc) +
+                          (neg ? values(std::false_type{}) : values(std::true_type{})));
+    __syncthreads();
     if (sl == 0) {
         uint64_t o = 0;
 #pragma unroll
