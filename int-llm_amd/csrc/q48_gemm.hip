@@ -1187,11 +1187,12 @@ __device__ __forceinline__ void win_sum128(const v16i (&acc)[11], int i, uint64_
 
 // grid (ceil(ceil(N/64) / NW) * ceil(T/64), 1, S) over operands split by
 // k_planes (nsteps k-steps): split z covers steps [z spb, (z + 1) spb), and a
-// block NW row tiles of W.  The block ORs its tiles' masks over its steps;
-// TOP is its W's top plane (at least 4); a block whose X digits reach plane 7
-// (or may overflow) or whose W digits leave TOP - 4 .. TOP writes nothing and
-// sets its tiles' redo flags (else clears them; the flag of a 64 x 64 tile is
-// that of its block in k_gemm_i8_full's numbering).  S == 1: Y gets the shifted
+// block NW row tiles of W.  The block ORs its tiles' masks over its steps; a
+// row tile's TOP is its top plane (at least 4).  A row tile whose digits leave
+// TOP - 4 .. TOP, and all of a block whose X digits reach plane 7 (or may
+// overflow), are not written and have their redo flags set (the others'
+// cleared; the flag of a 64 x 64 tile is that of its block in k_gemm_i8_full's
+// numbering).  S == 1: Y gets the shifted
 // result; S > 1: P[z][t][n] the int128 partial.  Row tiles whose planes are
 // shifted (prepared weights) give sums 2^shift too large: exact multiples,
 // shifted back.
@@ -1217,7 +1218,7 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
     __shared__ __align__(16) uint8_t st1[PSTAGE];
     __shared__ __align__(16) uint8_t st2[PSTAGE];
     __shared__ __align__(16) uint8_t st3[PSTAGE];
-    __shared__ uint32_t red[2][4];
+    __shared__ uint32_t red[1 + NW][4];
     // a byte per loop step, and the groups' words a group ahead
     constexpr int EXT_BYTES = 512;
     static_assert(MAXK_RUN / MK <= 510 && 256 * 2 == EXT_BYTES, "two steps a thread");
@@ -1239,7 +1240,7 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
     // which are still in L2.
     const bool rev = ((((int)blockIdx.x >> 3) / cpx) & 1) != 0;
     // the masks of loop steps tid and tid + 256 (ns <= 510)
-    uint32_t mx = 0, mw = 0, wk[2][NW];
+    uint32_t mx = 0, mw[NW] = {}, wk[2][NW];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         const int i = tid + 256 * u, k = s0 + (rev ? ns - 1 - i : i);
@@ -1254,22 +1255,38 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
     for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int j = 0; j < NW; ++j)
-            mw |= wk[u][j];
+            mw[j] |= wk[u][j];
     mx = wave_or(mx);
-    mw = wave_or(mw);
+#pragma unroll
+    for (int j = 0; j < NW; ++j)
+        mw[j] = wave_or(mw[j]);
     if (lane == 0) {
         red[0][w] = mx;
-        red[1][w] = mw;
+#pragma unroll
+        for (int j = 0; j < NW; ++j)
+            red[1 + j][w] = mw[j];
     }
     __syncthreads();
-    mx = (uint32_t)__builtin_amdgcn_readfirstlane((int)(red[0][0] | red[0][1] | red[0][2] | red[0][3]));
-    mw = (uint32_t)__builtin_amdgcn_readfirstlane((int)(red[1][0] | red[1][1] | red[1][2] | red[1][3]));
-    const int top = max((mw & 0xffu) ? 31 - __builtin_clz(mw & 0xffu) : 0, 4);
-    const uint32_t win = 0x1fu << (top - 4);
-    const bool fit = (mx & ~0x7fu) == 0 && (mw & ~win) == 0;
-    if (tid < NW && NW * n_blk + tid < nn)
-        redo[blockIdx.z * nn * nt + block_of(NW * n_blk + tid, t_tile, nn, nt)] = fit ? 0 : 1;
-    if (!fit) {
+    auto block_or = [&](int i) {
+        return (uint32_t)__builtin_amdgcn_readfirstlane(
+            (int)(red[i][0] | red[i][1] | red[i][2] | red[i][3]));
+    };
+    mx = block_or(0);
+    // Every row tile has its own window: with one for both, two of different
+    // magnitude would both be redone (1024 x 4096 x 2048 with every other row
+    // tile's weights 2^-24 of the rest: 430 us, now 204; equal ones 143)
+    int low[NW];   // TOP - 4
+    bool fit[NW], any = false;
+#pragma unroll
+    for (int j = 0; j < NW; ++j) {
+        mw[j] = block_or(1 + j);
+        low[j] = max((mw[j] & 0xffu) ? 31 - __builtin_clz(mw[j] & 0xffu) : 0, 4) - 4;
+        fit[j] = (mx & ~0x7fu) == 0 && (mw[j] & ~(0x1fu << low[j])) == 0;
+        any = any || fit[j];
+        if (tid == 0 && NW * n_blk + j < nn)
+            redo[blockIdx.z * nn * nt + block_of(NW * n_blk + j, t_tile, nn, nt)] = fit[j] ? 0 : 1;
+    }
+    if (!any) {
         wait_vm<0>();   // no DMA in flight when the block gives its LDS back
         return;         // uniform over the block
     }
@@ -1283,14 +1300,14 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
     const uint8_t *wsrc[NW];
 #pragma unroll
     for (int j = 0; j < NW; ++j)
-        wsrc[j] = Wp + ((size_t)n_tile[j] * nsteps + s0) * 8 * PLANE + (top - 4) * PLANE;
+        wsrc[j] = Wp + ((size_t)n_tile[j] * nsteps + s0) * 8 * PLANE + low[j] * PLANE;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         const int i = tid + 256 * u;
         uint32_t b = 0;
 #pragma unroll
         for (int j = 0; j < NW; ++j) {
-            const uint32_t m = wk[u][j] >> (top - 4);
+            const uint32_t m = fit[j] ? wk[u][j] >> low[j] : 0u;
             b |= ((m >> 1) & 1u) << j | (m & 1u) << 2;
         }
         if (i < EXT_BYTES)
@@ -1306,10 +1323,12 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
     const int wt = w >> 1, wn = w & 1;
 #pragma unroll
     for (int j = 0; j < NW; ++j) {
+        if (!fit[j])
+            continue;
         const int n = (NW * n_blk + j) * MN + 32 * wn + (lane & 31);
         const int t0 = t_tile * MT + 32 * wt + 4 * (lane >> 5);
         const int wsh = (int)((Wm[(size_t)n_tile[j] * nsteps] >> 16) & 7u);
-        const int sh = 48 + wsh - 8 * (top - 4);   // 24 .. 55
+        const int sh = 48 + wsh - 8 * low[j];   // 24 .. 55
         if (gridDim.z == 1) {
             int64_t y[16];
 #pragma unroll
@@ -1338,7 +1357,7 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
                 uint64_t lo, hi;
                 win_sum128(acc[j], i, lo, hi);
                 const q48_i128 u =
-                    (q48_i128)((((q48_u128)hi << 64) | lo) << (8 * (top - 4))) >> wsh;
+                    (q48_i128)((((q48_u128)hi << 64) | lo) << (8 * low[j])) >> wsh;
                 uint64_t *p = P + 2 * (((size_t)blockIdx.z * T + t) * N + n);
                 *reinterpret_cast<ulonglong2 *>(p) =
                     make_ulonglong2((uint64_t)u, (uint64_t)((q48_u128)u >> 64));
