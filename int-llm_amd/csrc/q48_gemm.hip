@@ -864,13 +864,14 @@ __device__ __forceinline__ void stage_barrier()
 // is unrolled by four), so the compiler's own waits for the reads of one
 // stage do not count the DMA into another.
 //
-// wsrc points at plane TOP - 4 of each row tile, and digit sums are kept
-// relative to it: acc[j][r] is the sum of weight 256^(TOP - 4 + r), so one code
+// wsrc points at plane TOP - 2 of each row tile (wext at TOP - 3, where there is
+// one), and digit sums are kept relative to TOP - 4, which may be below plane
+// 0: acc[j][r] is the sum of weight 256^(TOP - 4 + r), so one code
 // serves every window.  A step multiplies X planes 0..6 by W planes TOP - 2
 // .. TOP, 21 NW MFMAs, and by plane TOP - 3 only for a row tile that holds a
 // digit there (7 more; the shift of k_planes makes that about one step in ten
 // for bfloat16 weights).  ext (LDS) tells, a byte for each loop step, zero past
-// the last: bit n row tile n's plane TOP - 3, bit 2 some plane TOP - 4.  The
+// the last: bit n row tile n's plane TOP - 3, bit 2 + n its plane TOP - 4.  The
 // chunks of plane TOP - 3 are moved only then: otherwise their slots re-read a
 // fixed line set that stays in the vector cache, so that every step issues the
 // same number of DMAs with no branch around one, which would make the compiler
@@ -967,7 +968,9 @@ __device__ __forceinline__ void planes_pass(uint8_t (&s0)[stage_bytes(NW)],
                                             uint8_t (&s2)[stage_bytes(NW)],
                                             uint8_t (&s3)[stage_bytes(NW)],
                                             const uint8_t *ext, const uint8_t *xsrc,
-                                            const uint8_t *const (&wsrc)[NW], int ns, int xz,
+                                            const uint8_t *const (&wsrc)[NW],
+                                            const uint8_t *const (&wext)[NW],
+                                            const bool (&has5)[NW], int ns, int xz,
                                             bool rev, v16i (&acc)[NW][11])
 {
     constexpr int PSTAGE = stage_bytes(NW);
@@ -980,19 +983,24 @@ __device__ __forceinline__ void planes_pass(uint8_t (&s0)[stage_bytes(NW)],
     const int off = opnd_off(lane);
     // this wave's slot j moves chunk w + 4 j: its source in the first k-step (a
     // scalar address; the k-step's offset is one vector addition a step), and
-    // the ext bit it needs (0: none; 8: past the last chunk)
+    // the ext bit it needs (0: none; 16: past the last chunk)
     const uint8_t *base[CPW];
     uint32_t need[CPW];
 #pragma unroll
     for (int j = 0; j < CPW; ++j) {
         const int c = w + 4 * j, d = c - 14, x = c - DENSE;
         const uint8_t *wd = NW > 1 && d >= 6 ? wsrc[NW - 1] : wsrc[0];
-        const uint8_t *wx = NW > 1 && x >= 2 ? wsrc[NW - 1] : wsrc[0];
-        need[j] = c < DENSE ? 0u : c < ALL ? 1u << (x >> 1) : 8u;
+        const uint8_t *wx = NW > 1 && x >= 2 ? wext[NW - 1] : wext[0];
+        need[j] = c < DENSE ? 0u : c < ALL ? 1u << (x >> 1) : 16u;
         base[j] = c < 14 ? xsrc + c * 1024
-                  : c < DENSE ? wd + 2 * PLANE + (NW > 1 && d >= 6 ? d - 6 : d) * 1024
-                  : c < ALL ? wx + PLANE + (x & 1) * 1024 : xsrc;
+                  : c < DENSE ? wd + (NW > 1 && d >= 6 ? d - 6 : d) * 1024
+                  : c < ALL ? wx + (x & 1) * 1024 : xsrc;
     }
+    // plane TOP - 4, and TOP - 2 where there is none
+    const uint8_t *wlow[NW];
+#pragma unroll
+    for (int n = 0; n < NW; ++n)
+        wlow[n] = (has5[n] ? wsrc[n] - 2 * PLANE : wsrc[n]) + wn * SLICE + off;
     // Step s of the loop is k-step rev ? ns - 1 - s : s of the block's range.
     // The loop runs whole groups of four: steps past the last take the zero X
     // planes that follow the row tile's (k-step xz), with the last k-step of W.
@@ -1061,15 +1069,24 @@ __device__ __forceinline__ void planes_pass(uint8_t (&s0)[stage_bytes(NW)],
 #pragma unroll
                     for (int a = 0; a < 7; ++a)
                         mfma_i8(acc, n, a + 1, o.A[a], o.E[n]);
-            if (e & 4u)
+            if (e >> 2) {
+                // in bounds for every tile, used by those whose bit is set; the
+                // loads end in this branch, or the compiler waits for them, and
+                // for the DMAs, on the way without them too
+                v4i Bx[NW];
 #pragma unroll
-                for (int n = 0; n < NW; ++n) {
-                    const v4i Bx = *reinterpret_cast<const v4i *>(wsrc[n] + src_of(i).w +
-                                                                  wn * SLICE + off);
+                for (int n = 0; n < NW; ++n)
+                    Bx[n] = *reinterpret_cast<const v4i *>(wlow[n] + src_of(i).w);
 #pragma unroll
-                    for (int a = 0; a < 7; ++a)
-                        mfma_i8(acc, n, a, o.A[a], Bx);
-                }
+                for (int n = 0; n < NW; ++n)
+                    asm volatile("" : "+v"(Bx[n]));
+#pragma unroll
+                for (int n = 0; n < NW; ++n)
+                    if ((e >> (2 + n)) & 1u)
+#pragma unroll
+                        for (int a = 0; a < 7; ++a)
+                            mfma_i8(acc, n, a, o.A[a], Bx[n]);
+            }
             mfma_wait<NW>();
         }
         v4i nb[NW][3], a6;
@@ -1111,9 +1128,9 @@ __device__ __forceinline__ void planes_pass(uint8_t (&s0)[stage_bytes(NW)],
     // ext bits of loop steps i .. i + 3, from their bytes in a word
     auto ext4 = [&](uint32_t v, uint32_t &f0, uint32_t &f1, uint32_t &f2, uint32_t &f3) {
         const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
-        f0 = f & 7u;
-        f1 = (f >> 8) & 7u;
-        f2 = (f >> 16) & 7u;
+        f0 = f & 15u;
+        f1 = (f >> 8) & 15u;
+        f2 = (f >> 16) & 15u;
         f3 = f >> 24;
     };
     auto ext_word = [&](int i) { return *reinterpret_cast<const uint32_t *>(ext + i); };
@@ -1185,10 +1202,28 @@ __device__ __forceinline__ void win_sum128(const v16i (&acc)[11], int i, uint64_
     hi = (uint64_t)(g[0] >> 63) + (uint64_t)(g[1] >> 32) + carry + (uint64_t)g[2];
 }
 
+// Words of the signed 128-bit (lo, hi), Z zero words put below it, from bit b
+// (uniform, below 96) on, sign words above: word selects and funnel shifts.
+template <int N, int Z>
+__device__ __forceinline__ void words_from(uint64_t lo, uint64_t hi, int b, uint32_t (&o)[N])
+{
+    const uint32_t s = (uint32_t)((int64_t)hi >> 63);
+    const uint32_t w[8] = {(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi,
+                           (uint32_t)(hi >> 32), s, s, s, s};
+    const int q = b >> 5;
+    uint32_t a[N + 1];
+#pragma unroll
+    for (int k = 0; k <= N; ++k)
+        a[k] = q == 0 ? (k < Z ? 0u : w[k - Z]) : q == 1 ? w[k + 1 - Z] : w[k + 2 - Z];
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        o[k] = __builtin_amdgcn_alignbit(a[k + 1], a[k], b & 31);
+}
+
 // grid (ceil(ceil(N/64) / NW) * ceil(T/64), 1, S) over operands split by
 // k_planes (nsteps k-steps): split z covers steps [z spb, (z + 1) spb), and a
 // block NW row tiles of W.  The block ORs its tiles' masks over its steps; a
-// row tile's TOP is its top plane (at least 4).  A row tile whose digits leave
+// row tile's TOP is its top plane (at least 2).  A row tile whose digits leave
 // TOP - 4 .. TOP, and all of a block whose X digits reach plane 7 (or may
 // overflow), are not written and have their redo flags set (the others'
 // cleared; the flag of a 64 x 64 tile is that of its block in k_gemm_i8_full's
@@ -1275,13 +1310,14 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
     // Every row tile has its own window: with one for both, two of different
     // magnitude would both be redone (1024 x 4096 x 2048 with every other row
     // tile's weights 2^-24 of the rest: 430 us, now 204; equal ones 143)
-    int low[NW];   // TOP - 4
+    int low[NW];   // TOP - 4: -2 .. 3
     bool fit[NW], any = false;
 #pragma unroll
     for (int j = 0; j < NW; ++j) {
         mw[j] = block_or(1 + j);
-        low[j] = max((mw[j] & 0xffu) ? 31 - __builtin_clz(mw[j] & 0xffu) : 0, 4) - 4;
-        fit[j] = (mx & ~0x7fu) == 0 && (mw[j] & ~(0x1fu << low[j])) == 0;
+        low[j] = max((mw[j] & 0xffu) ? 31 - __builtin_clz(mw[j] & 0xffu) : 0, 2) - 4;
+        fit[j] = (mx & ~0x7fu) == 0 && mw[j] < 0x100u &&
+                 (mw[j] & ((1u << max(low[j], 0)) - 1u)) == 0;
         any = any || fit[j];
         if (tid == 0 && NW * n_blk + j < nn)
             redo[blockIdx.z * nn * nt + block_of(NW * n_blk + j, t_tile, nn, nt)] = fit[j] ? 0 : 1;
@@ -1297,25 +1333,30 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
 #pragma unroll
         for (int d = 0; d < 11; ++d)
             acc[j][d] = (v16i){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const uint8_t *wsrc[NW];
+    const uint8_t *wsrc[NW], *wext[NW];
+    bool has5[NW];
 #pragma unroll
-    for (int j = 0; j < NW; ++j)
-        wsrc[j] = Wp + ((size_t)n_tile[j] * nsteps + s0) * 8 * PLANE + low[j] * PLANE;
+    for (int j = 0; j < NW; ++j) {
+        wsrc[j] = Wp + ((size_t)n_tile[j] * nsteps + s0) * 8 * PLANE + (low[j] + 2) * PLANE;
+        wext[j] = wsrc[j] - (low[j] > -2 ? PLANE : 0);
+        has5[j] = low[j] >= 0;
+    }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         const int i = tid + 256 * u;
         uint32_t b = 0;
 #pragma unroll
         for (int j = 0; j < NW; ++j) {
-            const uint32_t m = fit[j] ? wk[u][j] >> low[j] : 0u;
-            b |= ((m >> 1) & 1u) << j | (m & 1u) << 2;
+            const uint32_t m = fit[j] ? (wk[u][j] << 2) >> (low[j] + 2) : 0u;   // from TOP - 4
+            b |= ((m >> 1) & 1u) << j | (m & 1u) << (2 + j);
         }
         if (i < EXT_BYTES)
             ext[i] = (uint8_t)b;
     }
     __syncthreads();
     if (ns > 0)   // an empty split has its X slots' zeros in flight: waited for below
-        planes_pass<NW>(st0, st1, st2, st3, ext, xsrc, wsrc, ns, nsteps - s0, rev, acc);
+        planes_pass<NW>(st0, st1, st2, st3, ext, xsrc, wsrc, wext, has5, ns, nsteps - s0, rev,
+                        acc);
     else
         wait_vm<0>();
     mfma_settle<NW>(acc);
@@ -1328,14 +1369,17 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
         const int n = (NW * n_blk + j) * MN + 32 * wn + (lane & 31);
         const int t0 = t_tile * MT + 32 * wt + 4 * (lane >> 5);
         const int wsh = (int)((Wm[(size_t)n_tile[j] * nsteps] >> 16) & 7u);
-        const int sh = 48 + wsh - 8 * low[j];   // 24 .. 55
+        // bits b .. b + 63 of the sum are bits 48 .. 111 of the result's
+        const int b = 48 + wsh - 8 * low[j];   // 24 .. 71
         if (gridDim.z == 1) {
             int64_t y[16];
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 uint64_t lo, hi;
                 win_sum128(acc[j], i, lo, hi);
-                y[i] = (int64_t)((lo >> sh) | (hi << (64 - sh)));
+                uint32_t o[2];
+                words_from<2, 0>(lo, hi, b, o);
+                y[i] = (int64_t)(((uint64_t)o[1] << 32) | o[0]);
             }
             int64_t *p = Y + (size_t)t0 * N + n;
             if ((t_tile + 1) * MT <= T && (NW * n_blk + j + 1) * MN <= N) {   // whole tile
@@ -1356,11 +1400,10 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
                     continue;
                 uint64_t lo, hi;
                 win_sum128(acc[j], i, lo, hi);
-                const q48_i128 u =
-                    (q48_i128)((((q48_u128)hi << 64) | lo) << (8 * low[j])) >> wsh;
+                uint32_t u[4];
+                words_from<4, 1>(lo, hi, b - 16, u);   // from a zero word on: 8 .. 55
                 uint64_t *p = P + 2 * (((size_t)blockIdx.z * T + t) * N + n);
-                *reinterpret_cast<ulonglong2 *>(p) =
-                    make_ulonglong2((uint64_t)u, (uint64_t)((q48_u128)u >> 64));
+                *reinterpret_cast<uint4 *>(p) = make_uint4(u[0], u[1], u[2], u[3]);
             }
         }
     }
