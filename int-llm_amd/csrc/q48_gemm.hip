@@ -816,16 +816,27 @@ __global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst, uint3
     uint8_t *p = dst + (size_t)blockIdx.x * 8 * PLANE + pc.off;
     uint32_t m = (big ? 0x100u : 0u) | (sh << 16) | (code << 20);
 #pragma unroll
-    for (int a = 0; a < 8; ++a) {
-        *reinterpret_cast<uint2 *>(p + a * PLANE) = d[a];
+    for (int a = 0; a < 8; ++a)
         m |= (d[a].x | d[a].y) != 0 ? 1u << a : 0u;
-    }
     m = wave_or(m);
     if ((tid & 63) == 0)
         red[tid >> 6] = m;
     __syncthreads();
+    m = (uint32_t)__builtin_amdgcn_readfirstlane((int)(red[0] | red[1] | red[2] | red[3]));
     if (tid == 0)
-        mask[(size_t)rt * nsteps + st] = red[0] | red[1] | red[2] | red[3];
+        mask[(size_t)rt * nsteps + st] = m;
+    // W planes that k_gemm_i8p never reads are not written: those above the row
+    // tile's top plane, and a plane without digits that lies three or more below
+    // this block's top.  (Planes TOP - 2 .. TOP are read always, TOP of a run of
+    // k-steps being at least each block's top and 2, lower ones where the mask
+    // has their bit.)  Of N(0, 0.02) bfloat16 weights 3 planes in 8 are left,
+    // which pays for k_tile_shift's pass over W.
+    const int own = (m & 0xffu) ? 31 - __builtin_clz(m & 0xffu) : 0;
+    const int hi = shifted ? max((int)(code >> 3), 2) : 7;
+#pragma unroll
+    for (int a = 0; a < 8; ++a)
+        if (pitch != nsteps || (a <= hi && (((m >> a) & 1u) || own < a + 3)))
+            *reinterpret_cast<uint2 *>(p + a * PLANE) = d[a];
 }
 
 // One LDS stage of the planes path, NW row tiles of W: X planes 0..6, then W
