@@ -1440,7 +1440,7 @@ int q48_gemm_auto_kernel(int T, int N, int K)
 // rounds, the second nearly empty, where the tiles divide badly: 128 tokens x
 // 2560 x 2048 took 320 blocks at S = 4, 52.8 us (38.7 prepared), and takes 240 at S
 // = 3, 38.7 us (30.5).
-int q48_gemm_i8_splits(int T, int N, int K, int cu_count, bool planes)
+static int i8_splits(int T, int N, int K, int cu_count, bool planes, int64_t *ns = nullptr)
 {
     const int64_t base = (int64_t)((N + MN - 1) / MN) * ((T + MT - 1) / MT);
     const int steps = (K + MK - 1) / MK;
@@ -1459,7 +1459,27 @@ int q48_gemm_i8_splits(int T, int N, int K, int cu_count, bool planes)
             best = s;
         }
     }
+    if (ns)
+        *ns = cost;
     return best;
+}
+
+// Whether splitting both operands into planes first pays for weights that are
+// not prepared, by the estimate above: the planes' k-steps are shorter, and
+// two launches (5.5 us) and 16 bytes a value at 5 TB/s come before them.
+// Measured (us, split in the loop / planes): 96 tokens x 11264 x 2048 120 /
+// 126, 128 x 2560 x 2048 37 / 42, 256 x 1024 x 1024 22 / 28, 2048 x 256 x 2048
+// 45 / 45; 160 x 11264 x 2048 197 / 163, 192 x 5632 x 2048 116 / 89, 256 x
+// 2560 x 2048 65 / 51, 2048 x 512 x 2048 69 / 57, 2048 x 11264 x 2048 1433 /
+// 820.  Over 150 shapes (64 to 2048 tokens, N 128 to 11264, K 256 to 5632) the choice
+// costs 0.25% on average and 10% at most over the better one; at least 256
+// tokens and N >= 1024, the line before, 2.5% and 30%.
+static bool planes_pay(int T, int N, int K, int cu_count)
+{
+    int64_t fused, planes;
+    i8_splits(T, N, K, cu_count, false, &fused);
+    i8_splits(T, N, K, cu_count, true, &planes);
+    return planes + 5500 + 16ll * ((int64_t)T + N) * K / 5000 < fused;
 }
 
 size_t q48_gemm_planes_size(int N, int K)
@@ -1487,40 +1507,47 @@ int q48_launch_gemm_i8(q48_ctx *c, int64_t *Y, const int64_t *W, const int64_t *
 {
     const int steps = (K + MK - 1) / MK;
     const int nt = (T + MT - 1) / MT, nn = (N + MN - 1) / MN, nb = nn * nt;
-    // the planes path pays one split of X (and of W unless prepared) per
-    // call: it wins once tiles are reused enough (measured: T >= 512 with
-    // N >= 2048 faster by 7-39%, N = 256 slower by 5-22%, T = 128 even when
-    // W is split in the call); with W prepared it wins from 2 tokens, where
-    // the GEMM streams W and the planes hold 5 of its 8 bytes per element
+    // with W prepared, planes win from 2 tokens on: the GEMM streams W then, and
+    // 3 to 4 planes hold a value's 8 bytes
     const bool fits = (size_t)max(nt, nn) * (steps + 1) <= 0x7fffffff;
-    const bool planes =
-        fits && (kernel == Q48_GEMM_I8_PLANES ||
-                 (kernel != Q48_GEMM_I8_FUSED && T >= (Wpre ? 2 : 256) && N >= 1024));
-    const bool wsplit = planes && !Wpre;
-    int S = q48_gemm_i8_splits(T, N, K, c->cu_count, planes);
-    int spb = (steps + S - 1) / S;
-    // planes_pass reaches a row tile's zero X planes by a 32-bit offset from
-    // the split's start.  Where that can pass 4 GB only the last split, which
-    // they follow directly, may need them: whole groups of four steps elsewhere
-    if (planes && (size_t)steps * 8 * PLANE > 0xffffffffu) {
-        spb = min((spb + 3) & ~3, MAXK_RUN / MK & ~3);
-        S = (steps + spb - 1) / spb;
-    }
-    // blocks (and their redo flags) are numbered in int
-    if ((size_t)((N + MN - 1) / MN) * ((T + MT - 1) / MT) * S > 0x7fffffff)
-        return Q48_EINVAL;
+    const bool choose =
+        fits && !Wpre && kernel != Q48_GEMM_I8_PLANES && kernel != Q48_GEMM_I8_FUSED;
+    bool planes = fits && (kernel == Q48_GEMM_I8_PLANES ||
+                           (kernel != Q48_GEMM_I8_FUSED && Wpre && T >= 2 && N >= 1024) ||
+                           (choose && planes_pay(T, N, K, c->cu_count)));
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    // workspace: the blocks' redo flags, (S > 1) the int128 partials, then
-    // (planes path) X and W digit planes and their masks
-    const size_t flags = al((size_t)nb * S * sizeof(int));
-    const size_t part = S > 1 ? 16 * (size_t)S * T * N : 0;
-    const size_t xpl = planes ? (size_t)nt * (steps + 1) * 8 * PLANE : 0;
-    const size_t wpl = wsplit ? (size_t)nn * steps * 8 * PLANE : 0;
-    const size_t xms = planes ? al((size_t)nt * steps * 4) : 0;
-    const size_t wms = wsplit ? al((size_t)nn * steps * 4) : 0;
-    int rc = q48_ws_reserve(c, flags + part + xpl + wpl + xms + wms);
-    if (rc)
-        return rc;
+    int S, spb, rc;
+    size_t flags, part, xpl, wpl, xms;
+    for (bool again = false;; again = true) {
+        S = i8_splits(T, N, K, c->cu_count, planes);
+        spb = (steps + S - 1) / S;
+        // planes_pass reaches a row tile's zero X planes by a 32-bit offset from
+        // the split's start.  Where that can pass 4 GB only the last split, which
+        // they follow directly, may need them: whole groups of four steps elsewhere
+        if (planes && (size_t)steps * 8 * PLANE > 0xffffffffu) {
+            spb = min((spb + 3) & ~3, MAXK_RUN / MK & ~3);
+            S = (steps + spb - 1) / spb;
+        }
+        // workspace: the blocks' redo flags, (S > 1) the int128 partials, then
+        // (planes path) X and W digit planes and their masks
+        flags = al((size_t)nb * S * sizeof(int));
+        part = S > 1 ? 16 * (size_t)S * T * N : 0;
+        xpl = planes ? (size_t)nt * (steps + 1) * 8 * PLANE : 0;
+        wpl = planes && !Wpre ? (size_t)nn * steps * 8 * PLANE : 0;
+        xms = planes ? al((size_t)nt * steps * 4) : 0;
+        const size_t wms = planes && !Wpre ? al((size_t)nn * steps * 4) : 0;
+        // blocks (and their redo flags) are numbered in int
+        rc = (size_t)nn * nt * S > 0x7fffffff
+                 ? Q48_EINVAL
+                 : q48_ws_reserve(c, flags + part + xpl + wpl + xms + wms);
+        if (!rc)
+            break;
+        // no room for the chosen form (nor, in a capture, a way to make some):
+        // the other one may fit
+        if (!choose || again)
+            return rc;
+        planes = !planes;
+    }
     char *ws = (char *)c->ws;
     int *redo = (int *)ws;
     uint64_t *P = S > 1 ? (uint64_t *)(ws + flags) : nullptr;

@@ -143,8 +143,6 @@ int q48_launch_gemm_i8(q48_ctx *c, int64_t *Y, const int64_t *W, const int64_t *
 // bytes of W's digit planes and masks for q48_launch_gemm_prepare
 size_t q48_gemm_planes_size(int N, int K);
 int q48_launch_gemm_prepare(q48_ctx *c, void *Wp, const int64_t *W, int N, int K);
-// K splits the int8 GEMM uses for this shape on cu_count compute units
-int q48_gemm_i8_splits(int T, int N, int K, int cu_count, bool planes);
 // Q48_GEMM_VALU or Q48_GEMM_I8: the kernel q48_gemm runs for this shape
 int q48_gemm_auto_kernel(int T, int N, int K);
 int q48_launch_rmsnorm(q48_ctx *c, int64_t *out, const int64_t *x,
