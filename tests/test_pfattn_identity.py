@@ -5,18 +5,26 @@ built on, checked by brute force with Python integers (no GPU):
    (mod 2^112), with S(v) the bytes of v ^ C as int8 except the top byte,
    also when some entries are the value C (all digits zero: pad positions
    and pad dims of the kernel);
-2. truncated products: sum_j floor(p_j v_j / 2^48)
-   = floor((sum_j p_j v_j - 2^24 sum_j t_j) / 2^48) (mod 2^64), t_j the
-   24-bit limb term (a0 b1 + a1 b0 + floor(a0 b0 / 2^24)) mod 2^24 of
-   a = p mod 2^48, b = v mod 2^48.
+2. truncated products: sum_j floor(p_j v_j / 2^48) as one FP64 sum rounding
+   down for values in [-2^51, 2^51), and as three such sums for any value,
+   v = v1 + 2^48 v2 (v1 = v mod 2^48), p = pa + 2^24 pb:
+   sum floor(p v1 / 2^48) + sum pa v2 + 2^24 sum pb v2, every sum within
+   2^51 of its start at the 4080 positions a wave has at most.
 
-A plausible slip (the top byte offset like the others, a dropped carry
-term, 2^24 t_j without the floor term) fails one of these cases.
+A plausible slip (the top byte offset like the others, rounding to nearest,
+the split left out for large values, more positions than the bound allows)
+fails one of these cases.
 """
 import random
+from fractions import Fraction
 
+from test_round_down_identity import fma, rd, rn
+
+ONE = 1 << 48
 C = 0x0080808080808080
 M24 = (1 << 24) - 1
+START = Fraction(3 << 51)          # Q48_FSUM0
+WAVE = 4080                        # positions a wave sums: 16320 / 4
 EDGE = [0, 1, -1, C, -(1 << 63), (1 << 63) - 1, 1 << 48, (1 << 48) - 1, -(1 << 48),
         1 << 24, (1 << 24) - 1, 0x7F7F7F7F7F7F7F7F, 0x8080808080808080 - (1 << 64)]
 
@@ -49,10 +57,36 @@ def digit_dot(xs, ws):
     return tot % (1 << 112)
 
 
-def t_term(p, v):
-    a, b = p & ((1 << 48) - 1), v & ((1 << 48) - 1)
-    a0, a1, b0, b1 = a & M24, a >> 24, b & M24, b >> 24
-    return (a0 * b1 + a1 * b0 + ((a0 * b0) >> 24)) & M24
+def fsum(ps, vs, r=rd):
+    """The wave's running FP64 sum of p v, p and v as the kernel holds them, and
+    the largest distance from its start."""
+    acc, far = START, 0
+    for p, v in zip(ps, vs):
+        acc = fma(p, v, acc, r)
+        far = max(far, abs(acc - START))
+    return int(acc - START), far
+
+
+def three_sums(ps, vs):
+    """q48_f51 of v's parts, the weights' parts from p 2^-48 (pass() in k_pfa)"""
+    scaled = [Fraction(p, ONE) for p in ps]
+    pb = [fma(p, 1 << 24, 1 << 52) - (1 << 52) for p in scaled]
+    pa = [fma(p, ONE, -b * (1 << 24)) for p, b in zip(scaled, pb)]
+    assert all(a + (int(b) << 24) == p and 0 <= a < 1 << 24 for a, b, p in zip(pa, pb, ps))
+    lo, hi = [v & (ONE - 1) for v in vs], [v >> 48 for v in vs]
+    parts = [fsum(scaled, lo), fsum(pa, hi), fsum(pb, hi)]
+    assert all(far <= 1 << 51 for _, far in parts)
+    return s64(parts[0][0] + parts[1][0] + (parts[2][0] << 24))
+
+
+def softmax_row(rng, n):
+    """n weights in [0, ONE] that add up to at most ONE"""
+    kind = rng.randrange(3)
+    if kind == 0:
+        return [ONE // n] * n
+    cut = sorted(rng.randrange(0, ONE + 1) for _ in range(n))
+    ps = [b - a for a, b in zip([0] + cut, cut)]
+    return ps if kind == 1 else [p >> rng.choice([0, 0, 30]) for p in ps]
 
 
 def draw(rng, edge_share=0.3):
@@ -81,23 +115,45 @@ def test_digit_identity_all_min():
     assert digit_dot(xs, xs) == sum(x * x for x in xs) % (1 << 112)
 
 
-def test_truncated_product_sum():
+def test_value_sums_in_range():
     rng = random.Random(1)
-    for trial in range(600):
+    edge = [-(1 << 51), (1 << 51) - 1, 0, -1, 1, ONE, -ONE]
+    nearest_differs = 0
+    for trial in range(120):
         n = rng.choice([1, 2, 3, 17, 64, 300])
-        ps = [rng.choice([rng.randrange(0, 1 << 49), rng.randrange(0, 1 << 63), 0, 1 << 48,
-                          (1 << 48) - 1, (1 << 24) - 1]) for _ in range(n)]
+        ps = softmax_row(rng, n)
+        vs = [rng.choice(edge) if trial % 3 == 0 else rng.randrange(-(1 << 51), 1 << 51)
+              for _ in range(n)]
+        want = sum(p * v >> 48 for p, v in zip(ps, vs))
+        scaled = [Fraction(p, ONE) for p in ps]
+        got, far = fsum(scaled, vs)
+        assert got == want and far <= 1 << 51, trial
+        nearest_differs += fsum(scaled, vs, rn)[0] != want
+    assert nearest_differs > 30
+
+
+def test_value_sums_of_any_value():
+    rng = random.Random(4)
+    whole_differs = 0
+    for trial in range(120):
+        n = rng.choice([1, 2, 3, 17, 64, 300])
+        ps = softmax_row(rng, n)
         vs = [draw(rng) for _ in range(n)]
-        want = s64(sum((p * v) >> 48 for p, v in zip(ps, vs)))
-        X = sum(p * v for p, v in zip(ps, vs)) % (1 << 112)
-        lam = sum(t_term(p, v) for p, v in zip(ps, vs))
-        assert s64((X - (lam << 24)) >> 48) == want, trial
+        want = s64(sum(p * v >> 48 for p, v in zip(ps, vs)))
+        assert three_sums(ps, vs) == want, trial
+        whole_differs += s64(fsum([Fraction(p, ONE) for p in ps],
+                                  [rd(Fraction(v)) for v in vs])[0]) != want
+    assert whole_differs > 60
 
 
-def test_truncated_product_needs_the_carry_term():
-    """dropping floor(a0 b0 / 2^24) from t_j gives a different sum"""
-    p, v = (1 << 48) - 1, (1 << 48) - 1
-    t_bad = (((p & M24) * (v >> 24 & M24)) + ((p >> 24 & M24) * (v & M24))) & M24
-    X = p * v
-    assert s64((X - (t_term(p, v) << 24)) >> 48) == s64((p * v) >> 48)
-    assert s64((X - (t_bad << 24)) >> 48) != s64((p * v) >> 48)
+def test_value_sums_at_the_longest_row():
+    """Equal weights whose low 24 bits are nearly all ones, values at both ends of
+    int64, as many positions as a wave sums: the low part comes to 0.96 of its
+    bound, and 4400 positions would leave it."""
+    p = ONE // 16305
+    assert p & M24 > 0.96 * (1 << 24)
+    for v in (-(1 << 63), -(1 << 63) + 1, (1 << 63) - 1):
+        assert three_sums([p] * WAVE, [v] * WAVE) == s64(WAVE * (p * v >> 48))
+    assert fsum([p & M24] * WAVE, [-(1 << 15)] * WAVE)[1] > 0.95 * (1 << 51)
+    n = 4400
+    assert fsum([p & M24] * n, [-(1 << 15)] * n)[1] > 1 << 51
