@@ -1216,6 +1216,12 @@ static int p6_grid(const q48_ctx *c, int groups)
     return (groups + rounds - 1) / rounds;
 }
 
+// 16-element tiles of a wave's segment for the K that have an unrolled instance
+// (eight waves, whole tiles), 0 for any other.  Two are instantiated, the row
+// lengths of the TinyLlama shape; other K, also of whole tiles, take the
+// batched loop or k_gemv_d.
+constexpr int v4_tiles(int K) { return K == 8 * 16 * 16 ? 16 : K == 8 * 16 * 44 ? 44 : 0; }
+
 template <int PRO, int EPI>
 static int launch_v4(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
                      const int64_t *norm_w, const int64_t *r_in, int64_t *r_out, int M, int K,
@@ -1232,16 +1238,15 @@ static int launch_v4(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
         if (rc)
             return rc;
     }
-    // K = 2048 and K = 5632 (every wave: 16 or 44 whole tiles) take the
-    // unrolled rotating pipeline; other K the batched loop
+    // the unrolled rotating pipeline where K has one; other K the batched loop
     const bool al = (((uintptr_t)W | (uintptr_t)x) & 15) == 0 &&
                     (PRO == 0 || ((uintptr_t)norm_w & 15) == 0) &&
                     (PRO != 3 || ((uintptr_t)r_in & 15) == 0);
+    const int tiles = al ? v4_tiles(K) : 0;
     // more row groups than two rounds of blocks: the persistent form
     if constexpr ((PRO == 0 || PRO == 3) && (EPI == 0 || EPI == 2)) {
         const int grid = 2 * c->cu_count;
-        if (al && K == NW * seg && seg == 16 * 16 && blocks > 2 * grid &&
-            blocks <= P6_MAXG * grid && c->gemv_persistent) {
+        if (tiles == 16 && blocks > 2 * grid && blocks <= P6_MAXG * grid && c->gemv_persistent) {
             hipLaunchKernelGGL((k_gemv_p6<NW, 4, PRO, EPI, 16>), dim3(p6_grid(c, blocks)),
                                dim3(64 * NW), lds,
                                c->stream, y, W, x, norm_w, r_in, M, K, seg);
@@ -1259,11 +1264,11 @@ static int launch_v4(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
             return (int)hipGetLastError();
         }
     }
-    if (al && K == NW * seg && seg == 16 * 16)
+    if (tiles == 16)
         hipLaunchKernelGGL((k_gemv_v5<NW, 4, PRO, EPI, 16>), dim3(blocks), dim3(64 * NW), lds,
                            c->stream, y, W, x, norm_w, r_in, r_out, c->rms_part, c->rms_count,
                            M, K, seg, rkv);
-    else if (al && K == NW * seg && seg == 16 * 44)
+    else if (tiles == 44)
         hipLaunchKernelGGL((k_gemv_v5<NW, 6, PRO, EPI, 44>), dim3(blocks), dim3(64 * NW), lds,
                            c->stream, y, W, x, norm_w, r_in, r_out, c->rms_part, c->rms_count,
                            M, K, seg, rkv);
@@ -1616,11 +1621,11 @@ int q48_launch_rms_apply(q48_ctx *c, int64_t *out, const int64_t *x, const int64
 int q48_launch_gemv(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
                     int M, int K)
 {
-    // the decode kernel where its tiles come out whole, the direct one
+    // the decode kernel where it is unrolled for K, the direct one
     // elsewhere (us, direct against k_gemv_v5's batched loop: 1376 x 256 4.6 /
     // 5.5, 4096 x 4096 24.9 / 28.5, 64 x 8191 5.7 / 22.6, 5632 x 1999 19.6 /
     // 21.9; but 1031 x 2048 7.4 / 5.7 with whole tiles)
-    if ((K == 2048 || K == 5632) && (((uintptr_t)W | (uintptr_t)x) & 15) == 0)
+    if (v4_tiles(K) > 0 && (((uintptr_t)W | (uintptr_t)x) & 15) == 0)
         return launch_v4<0, 0>(c, y, W, x, nullptr, nullptr, nullptr, M, K);
     // waves per row: until 2048 waves (8 a compute unit) or one tile each;
     // many short rows: four a wave, for the loads in flight and x read once.
