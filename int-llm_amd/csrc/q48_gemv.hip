@@ -63,7 +63,7 @@ __device__ __forceinline__ q48_u128 acc_value(const LimbAcc &A)
 // k_gemv_d: any K and 8-byte alignment.  S waves share a row (1, 2, 4 or 8: 8 / S
 // rows a block), or a wave takes RW rows (S = 1).  A wave's segment streams as
 // 1 KB tiles (lane l: elements 2 l, 2 l + 1; 16-byte loads, which take any dword
-// alignment, so odd K costs nothing), UNR of each row in flight together with
+// alignment), UNR of each row in flight together with
 // the same elements of x from the cache: nothing is staged and no barrier comes
 // before the loads, at the price of x read once per wave.  The segment's last,
 // partial tile goes out with the first batch.
@@ -107,27 +107,59 @@ __global__ __launch_bounds__(512) void k_gemv_d(int64_t *__restrict__ y,
             te[r][e] = in ? (uint64_t)wr[r][128 * nt + 2 * lane + e] : 0;
     }
     const v2u *x2 = reinterpret_cast<const v2u *>(xr) + lane;
-    for (int t0 = 0; t0 < nt; t0 += UNR) {
-        v2u wv[RW][UNR], xv[UNR];
+    auto load = [&](v2u &wv, int r, int t) {
+        wv = __builtin_nontemporal_load(reinterpret_cast<const v2u *>(wr[r]) + lane + 64 * t);
+    };
+    auto tile = [&](const v2u (&wv)[RW], v2u xv) {
+#pragma unroll
+        for (int r = 0; r < RW; ++r) {
+            mac(A[r], xv.x, wv[r].x);
+            mac(A[r], xv.y, wv[r].y);
+        }
+        xsum += xv.x + xv.y;
+    };
+    // Whole batches, then the tiles that are left.  Four rows a wave, two tiles a
+    // batch: a batch with its last tile loaded twice (fewer registers; 32000 x
+    // 256 14.0 us, 14.5 with the other form).  One row a wave: by the bits of
+    // their number (repeated tiles took 3000 x 511 4.9 us, now 4.0, 16384 x 700
+    // 22.4, now 17.4, 6000 x 4095 35.5, now 33.7).
+    int t0 = 0;
+    for (; t0 + (RW > 1 ? 1 : UNR) <= nt; t0 += UNR) {
+        v2u wv[UNR][RW], xv[UNR];
 #pragma unroll
         for (int u = 0; u < UNR; ++u)
 #pragma unroll
             for (int r = 0; r < RW; ++r)
-                wv[r][u] = __builtin_nontemporal_load(reinterpret_cast<const v2u *>(wr[r]) + lane +
-                                                      64 * min(t0 + u, nt - 1));
+                load(wv[u][r], r, RW > 1 ? min(t0 + u, nt - 1) : t0 + u);
 #pragma unroll
         for (int u = 0; u < UNR; ++u)
-            xv[u] = x2[64 * min(t0 + u, nt - 1)];
+            xv[u] = x2[64 * (RW > 1 ? min(t0 + u, nt - 1) : t0 + u)];
 #pragma unroll
         for (int u = 0; u < UNR; ++u)
-            if (t0 + u < nt) {
+            if (RW == 1 || t0 + u < nt)
+                tile(wv[u], xv[u]);
+    }
+    if (RW == 1 && t0 < nt) {
+        v2u wv[UNR][RW], xv[UNR];
+        int t = t0, u0 = 0;
 #pragma unroll
-                for (int r = 0; r < RW; ++r) {
-                    mac(A[r], xv[u].x, wv[r][u].x);
-                    mac(A[r], xv[u].y, wv[r][u].y);
+        for (int n = UNR / 2; n >= 1; n /= 2, u0 += 2 * n) {
+            if ((nt - t0) & n) {
+#pragma unroll
+                for (int u = 0; u < n; ++u) {
+                    load(wv[u0 + u][0], 0, t + u);
+                    xv[u0 + u] = x2[64 * (t + u)];
                 }
-                xsum += xv[u].x + xv[u].y;
+                t += n;
             }
+        }
+        u0 = 0;
+#pragma unroll
+        for (int n = UNR / 2; n >= 1; n /= 2, u0 += 2 * n)
+            if ((nt - t0) & n)
+#pragma unroll
+                for (int u = 0; u < n; ++u)
+                    tile(wv[u0 + u], xv[u0 + u]);
     }
     xsum += xe[0] + xe[1];
 #pragma unroll
