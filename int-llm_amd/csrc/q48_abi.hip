@@ -648,24 +648,48 @@ bool meets(Words a, Words b)
            (uintptr_t)b.p < (uintptr_t)(a.p + a.n);
 }
 
+// Where a fused GEMV on rows that start on 8 bytes (odd K, or W itself) stays one
+// launch: up to `rows` rows with K <= 1024 (the short-row kernels), up to `words`
+// weights with K <= 2048, nowhere above.  Its loads of unaligned rows touch more
+// lines than k_gemv_d's, so from some size on the separate launches win, the
+// later the more of them there are.  us, one launch / separate, at 600, 4002 and
+// 11262 rows of K = 1025:
+//   norm_gemv_stats         10.8 / 10.8   17.1 / 11.3   41.5 / 21.0
+//   norm_gemv_swiglu_stats   9.7 / 14.0   18.0 / 14.6   44.1 / 23.7
+//   gemv_residual            7.0 /  7.8   11.6 /  8.7   31.9 / 18.7
+// and of K = 511 5.1 / 11.0, 6.0 / 10.7, 12.3 / 16.2 (norm_gemv_stats); 4095:
+// 18.6 / 12.4, 35.4 / 28.3, 98.5 / 69.5.
+struct Unaligned {
+    int rows;
+    size_t words;
+};
+constexpr Unaligned kUnNorm = {8192, 0}, kUnNormStats = {8192, 5 << 17}, kUnOwnNorm = {4096, 0};
+constexpr Unaligned kUnSwiglu = {8192, 2 << 20}, kUnSwigluStats = {8192, 4 << 20};
+constexpr Unaligned kUnOwnNormSwiglu = {8192, 8 << 20};
+constexpr Unaligned kUnResidual = {8192, 5 << 18}, kUnResidualStats = {8192, 4 << 20};
+constexpr Unaligned kUnResidualRms = {2048, 0};
+
 // Whether a GEMV and what surrounds it may be one launch.  Its blocks write
 // their rows while others still read the vectors, so an output that shares
 // words with one of them takes the separate launches, which go through a
-// temporary.  (A single block reads all it needs before it writes; with even K
-// and aligned W such a call stays one launch, which needs no temporary, as a
-// capture may demand.)
-bool one_launch(const int64_t *W, int M, int K, std::initializer_list<Words> out,
-                std::initializer_list<Words> in)
+// temporary of tmp words.  (A single block reads all it needs before it writes;
+// with even K and aligned W such a call stays one launch, which needs no
+// temporary, as a capture may demand.)  A capture that cannot make the
+// temporary takes one launch wherever it may.
+bool one_launch(const q48_ctx *c, const int64_t *W, int M, int K, Unaligned un, size_t tmp,
+                std::initializer_list<Words> out, std::initializer_list<Words> in)
 {
     if (!q48_gemv_v5_ok(M, K))
         return false;
-    if (M <= 8 && q48_gemv_v2_ok(W, K))
+    const bool aligned = q48_gemv_v2_ok(W, K);
+    if (M <= 8 && aligned)
         return true;
     for (const Words &o : out)
         for (const Words &i : in)
             if (meets(o, i))
                 return false;
-    return true;
+    return aligned || (K <= 1024 ? M <= un.rows : K <= 2048 && (size_t)M * K <= un.words) ||
+           (c->capturing && c->tmp_bytes < tmp * 8);
 }
 } // namespace
 
@@ -674,7 +698,8 @@ int q48_rmsnorm_gemv(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
 {
     if (!c || bad_ptrs(y, W, x) || !norm_w || M <= 0 || K <= 0 || M > kMaxDim || K > kMaxDim)
         return Q48_EINVAL;
-    if (one_launch(W, M, K, {{y, (size_t)M}}, {{x, (size_t)K}, {norm_w, (size_t)K}})) {
+    if (one_launch(c, W, M, K, kUnOwnNorm, (size_t)K,
+                   {{y, (size_t)M}}, {{x, (size_t)K}, {norm_w, (size_t)K}})) {
         int prc;
         q48_ctx::ProfRec *r = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -694,7 +719,8 @@ int q48_gemv_residual(q48_ctx *c, int64_t *acc, const int64_t *W, const int64_t 
 {
     if (!c || bad_ptrs(acc, W, x) || M <= 0 || K <= 0 || M > kMaxDim || K > kMaxDim)
         return Q48_EINVAL;
-    if (one_launch(W, M, K, {{acc, (size_t)M}}, {{x, (size_t)K}})) {
+    if (one_launch(c, W, M, K, kUnResidual, (size_t)M,
+                   {{acc, (size_t)M}}, {{x, (size_t)K}})) {
         int prc;
         q48_ctx::ProfRec *r = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -715,7 +741,8 @@ int q48_rmsnorm_gemv_swiglu(q48_ctx *c, int64_t *out, const int64_t *Wgu, const 
     if (!c || bad_ptrs(out, Wgu, x) || !norm_w || ffn <= 0 || K <= 0 || ffn > kMaxDim / 2 ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (one_launch(Wgu, 2 * ffn, K, {{out, (size_t)ffn}},
+    if (one_launch(c, Wgu, 2 * ffn, K, kUnOwnNormSwiglu, (size_t)K + 2 * (size_t)ffn,
+                   {{out, (size_t)ffn}},
                    {{x, (size_t)K}, {norm_w, (size_t)K}})) {
         int prc;
         q48_ctx::ProfRec *r = prof_begin(c, gemv_bytes(2 * ffn, K, ffn), &prc);
@@ -947,7 +974,8 @@ int q48_norm_gemv(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t *x,
     if (!c || bad_ptrs(y, W, x) || !norm_w || !r || M <= 0 || K <= 0 || M > kMaxDim ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (one_launch(W, M, K, {{y, (size_t)M}}, {{x, (size_t)K}, {norm_w, (size_t)K}, {r, 1}})) {
+    if (one_launch(c, W, M, K, kUnNorm, (size_t)K,
+                   {{y, (size_t)M}}, {{x, (size_t)K}, {norm_w, (size_t)K}, {r, 1}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -969,7 +997,8 @@ int q48_norm_gemv_swiglu(q48_ctx *c, int64_t *out, const int64_t *Wgu, const int
     if (!c || bad_ptrs(out, Wgu, x) || !norm_w || !r || ffn <= 0 || K <= 0 ||
         ffn > kMaxDim / 2 || K > kMaxDim)
         return Q48_EINVAL;
-    if (one_launch(Wgu, 2 * ffn, K, {{out, (size_t)ffn}},
+    if (one_launch(c, Wgu, 2 * ffn, K, kUnSwiglu, (size_t)K + 2 * (size_t)ffn,
+                   {{out, (size_t)ffn}},
                    {{x, (size_t)K}, {norm_w, (size_t)K}, {r, 1}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(2 * ffn, K, ffn), &prc);
@@ -994,7 +1023,8 @@ int q48_gemv_residual_rms(q48_ctx *c, int64_t *acc, const int64_t *W, const int6
     if (!c || bad_ptrs(acc, W, x) || !r_out || M <= 0 || K <= 0 || M > kMaxDim ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (one_launch(W, M, K, {{acc, (size_t)M}, {r_out, 1}}, {{x, (size_t)K}})) {
+    if (one_launch(c, W, M, K, kUnResidualRms, (size_t)M,
+                   {{acc, (size_t)M}, {r_out, 1}}, {{x, (size_t)K}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
         if (prc)
@@ -1045,7 +1075,8 @@ int q48_norm_gemv_stats(q48_ctx *c, int64_t *y, const int64_t *W, const int64_t 
     if (!c || bad_ptrs(y, W, x) || !norm_w || !stats || M <= 0 || K <= 0 || M > kMaxDim ||
         K > kMaxDim)
         return Q48_EINVAL;
-    if (one_launch(W, M, K, {{y, (size_t)M}},
+    if (one_launch(c, W, M, K, kUnNormStats, (size_t)K,
+                   {{y, (size_t)M}},
                    {{x, (size_t)K}, {norm_w, (size_t)K}, {stats, (size_t)Q48_STATS_WORDS(K)}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
@@ -1065,7 +1096,8 @@ int q48_norm_gemv_swiglu_stats(q48_ctx *c, int64_t *out, const int64_t *Wgu, con
     if (!c || bad_ptrs(out, Wgu, x) || !norm_w || !stats || ffn <= 0 || K <= 0 ||
         ffn > kMaxDim / 2 || K > kMaxDim)
         return Q48_EINVAL;
-    if (one_launch(Wgu, 2 * ffn, K, {{out, (size_t)ffn}},
+    if (one_launch(c, Wgu, 2 * ffn, K, kUnSwigluStats, (size_t)K + 2 * (size_t)ffn,
+                   {{out, (size_t)ffn}},
                    {{x, (size_t)K}, {norm_w, (size_t)K}, {stats, (size_t)Q48_STATS_WORDS(K)}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(2 * ffn, K, ffn), &prc);
@@ -1084,7 +1116,8 @@ int q48_gemv_residual_stats(q48_ctx *c, int64_t *acc, const int64_t *W, const in
 {
     if (!c || bad_ptrs(acc, W, x) || !stats || M <= 0 || K <= 0 || M > kMaxDim || K > kMaxDim)
         return Q48_EINVAL;
-    if (one_launch(W, M, K, {{acc, (size_t)M}, {stats, (size_t)Q48_STATS_WORDS(M)}},
+    if (one_launch(c, W, M, K, kUnResidualStats, (size_t)M,
+                   {{acc, (size_t)M}, {stats, (size_t)Q48_STATS_WORDS(M)}},
                    {{x, (size_t)K}})) {
         int prc;
         q48_ctx::ProfRec *pr = prof_begin(c, gemv_bytes(M, K, M), &prc);
