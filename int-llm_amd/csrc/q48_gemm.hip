@@ -1247,11 +1247,11 @@ __device__ __forceinline__ void words_from(uint64_t lo, uint64_t hi, int b, uint
 // step moves 26 KB for 42 MFMAs a wave, where NW = 1 moves 20 KB for 21.
 //
 // What bounds it: the matrix cores at the clock their power allows.  A loop of
-// nothing but these MFMAs on random digits runs at 3.3 POP/s (4.5-4.9 on
+// nothing but these MFMAs on random digits runs at 3.1 to 3.5 POP/s (4.3-4.8 on
 // zeros); 2048 x 11264 x 2048 takes 22 digit products per Q16.48 MAC here, 2.8
-// POP/s over its 745 us.  With a four-plane window always multiplied (28
-// products), the DMA ahead of the MFMAs and a 64-bit vector address per chunk
-// the call took 991 us on the same card (776 now with the split of X).
+// POP/s over 735 us, with the matrix cores busy two thirds of the time at 1.75
+// GHz.  With a four-plane window always multiplied (28 products), the DMA ahead
+// of the MFMAs and a 64-bit vector address per chunk the call took 931 us.
 template <int NW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ redo,
@@ -1364,6 +1364,8 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
         if (i < EXT_BYTES)
             ext[i] = (uint8_t)b;
     }
+    if (tid < 3)   // the words read a group ahead, past the last step
+        reinterpret_cast<uint32_t *>(ext + EXT_BYTES)[tid] = 0;
     __syncthreads();
     if (ns > 0)   // an empty split has its X slots' zeros in flight: waited for below
         planes_pass<NW>(st0, st1, st2, st3, ext, xsrc, wsrc, wext, has5, ns, nsteps - s0, rev,
@@ -1568,16 +1570,16 @@ int q48_launch_gemm_i8(q48_ctx *c, int64_t *Y, const int64_t *W, const int64_t *
                                K, steps, steps, 0);
         }
         // one or two row tiles a block, by rounds of blocks over the compute
-        // units: a block of two takes 1.93 times one of one (2048 x 11264 x
-        // 2048: 22 rounds in 806 us, 11 in 776), so two win where they need
-        // half the rounds (or a little over half, with many), and lose where
-        // the last round is emptier (2048 x 2048, 1500 tokens: 3 rounds 121
-        // us, 2 rounds 136).  Split K keeps one: its runs are short, and the
-        // part that fills the device is what it is for (128 tokens x 2560 x
-        // 2048: 39.0 against 41.6 us).
+        // units: a block of two takes 1.78 to 1.87 times one of one (2048 x 11264
+        // x 2048: 22 rounds in 794 us, 11 in 740), so two win from 11 rounds
+        // against 6 on (us, one / two: 11 and 6 rounds 396 / 385, 17 and 9 592 /
+        // 572, 19 and 10 672 / 643), and lose where the last round is emptier
+        // (7 and 4 252 / 255, 3 and 2 123 / 136).  Split K keeps one: its runs
+        // are short, and the part that fills the device is what it is for (128
+        // tokens x 2560 x 2048: 39.0 against 41.6 us).
         const int cu = c->cu_count, cpx = max(1, cu / 8), nb2 = (nn + 1) / 2 * nt;
         const int rounds1 = (nb + cu - 1) / cu, rounds2 = (nb2 + cu - 1) / cu;
-        if (S == 1 && 29 * rounds2 <= 15 * rounds1)
+        if (S == 1 && 11 * rounds2 <= 6 * rounds1)
             hipLaunchKernelGGL(k_gemm_i8p<2>, dim3(nb2, 1, 1), dim3(256), 0, c->stream, Y, P,
                                redo, Xp, Xm, Wp, Wm, T, N, steps, spb, cpx);
         else
