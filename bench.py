@@ -171,9 +171,10 @@ def gemm_prefill(ctx, spec, intllm, reps: int):
                         "bf16-exact, X N(0,1) raw Q16.48",
             "i8_peak_ops": I8_PEAK_OPS, "i8_ops_per_mac": I8_OPS_PER_MAC,
             "i8_frac_basis": "63 int8 digit products (126 ops) per Q16.48 MAC, the full "
-                             "digit expansion; for these bfloat16-exact weights the kernel "
-                             "runs 28-35 of them (zero digit planes skipped), so i8_frac "
-                             "is the rate on the algorithmic count, not MFMA occupancy",
+                             "digit expansion; for these bfloat16-exact weights the planes "
+                             "kernel runs 21-28 of them and the in-loop split 28-35 (zero "
+                             "digit planes skipped), so i8_frac is the rate on the "
+                             "algorithmic count, not MFMA occupancy",
             "valu_mad_peak": VALU_MAD_PEAK, "valu_mads_per_mac": VALU_MADS_PER_MAC,
             "shapes": out}
 
