@@ -741,24 +741,25 @@ __global__ __launch_bounds__(1024) void k_tile_shift(uint32_t *__restrict__ mask
 // past R and columns past K are zero), and mask[rt * nsteps + s] has bit a
 // when plane a holds a nonzero digit and bit 8 when a value may have
 // overflowed v + C (high word >= 0x7F7F7F7F; plane 8 itself is not stored).
-// pitch: blocks per row tile, one past nsteps holding zero planes (X: nsteps + 1,
-// for the steps that fill up the k loop's groups of four; W: nsteps).
-// shifted: the row tile's values are multiplied by 2^shift before the split
+// X (!WGT) has one block more per row tile, of zero planes, for the steps that fill
+// up the k loop's groups of four.
+// shifted (WGT): the row tile's values are multiplied by 2^shift before the split
 // (from the largest code of k_tile_shift's parts; every mask of the row tile
 // keeps that code, so a block may read a part's word before or after the
 // block that writes its own mask there; bits 16..18: the shift), so that the largest one fills its top plane: a
 // bfloat16 weight's low bits then reach down to fewer planes (N(0, 0.02)
 // weights: 10% of the 64 x 32 tiles need a fourth plane, 34% unshifted).
+template <bool WGT>
 __global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst, uint32_t *mask,
                                                const int64_t *__restrict__ src, int R, int K,
-                                               int nsteps, int pitch, int shifted)
+                                               int nsteps, int shifted)
 {
     __shared__ uint32_t red[4];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, pitch = WGT ? nsteps : nsteps + 1;
     const int rt = (int)blockIdx.x / pitch, st = (int)blockIdx.x % pitch;
     const Piece pc = piece(tid);
     const int row = rt * MN + pc.r, k0 = st * MK + pc.k8;
-    if (st >= nsteps) {   // padding: zero planes, no mask
+    if (!WGT && st >= nsteps) {   // padding: zero planes, no mask
         for (int i = tid; i < PLANE / 2; i += 256)
             reinterpret_cast<uint4 *>(dst + (size_t)blockIdx.x * 8 * PLANE)[i] =
                 make_uint4(0, 0, 0, 0);
@@ -780,7 +781,7 @@ __global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst, uint3
             v[e] = row < R && k0 + e < K ? (uint64_t)rp[e] : 0;
     }
     uint32_t sh = 0, code = 0;
-    if (shifted) {
+    if (WGT && shifted) {
         const int part = min(tid & (TS_PARTS - 1), tile_parts(K, nsteps) - 1);
         code = (__hip_atomic_load(mask + (size_t)rt * nsteps + part, __ATOMIC_RELAXED,
                                   __HIP_MEMORY_SCOPE_AGENT) >> 20) & 63u;
@@ -816,12 +817,20 @@ __global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst, uint3
     uint8_t *p = dst + (size_t)blockIdx.x * 8 * PLANE + pc.off;
     uint32_t m = (big ? 0x100u : 0u) | (sh << 16) | (code << 20);
 #pragma unroll
-    for (int a = 0; a < 8; ++a)
+    for (int a = 0; a < 8; ++a) {
+        if (!WGT)   // every plane, without waiting for the mask
+            *reinterpret_cast<uint2 *>(p + a * PLANE) = d[a];
         m |= (d[a].x | d[a].y) != 0 ? 1u << a : 0u;
+    }
     m = wave_or(m);
     if ((tid & 63) == 0)
         red[tid >> 6] = m;
     __syncthreads();
+    if constexpr (!WGT) {
+        if (tid == 0)
+            mask[(size_t)rt * nsteps + st] = red[0] | red[1] | red[2] | red[3];
+        return;
+    }
     m = (uint32_t)__builtin_amdgcn_readfirstlane((int)(red[0] | red[1] | red[2] | red[3]));
     if (tid == 0)
         mask[(size_t)rt * nsteps + st] = m;
@@ -835,7 +844,7 @@ __global__ __launch_bounds__(256) void k_planes(uint8_t *__restrict__ dst, uint3
     const int hi = shifted ? max((int)(code >> 3), 2) : 7;
 #pragma unroll
     for (int a = 0; a < 8; ++a)
-        if (pitch != nsteps || (a <= hi && (((m >> a) & 1u) || own < a + 3)))
+        if (a <= hi && (((m >> a) & 1u) || own < a + 3))
             *reinterpret_cast<uint2 *>(p + a * PLANE) = d[a];
 }
 
@@ -1331,7 +1340,9 @@ k_gemm_i8p(int64_t *__restrict__ Y, uint64_t *__restrict__ P, int *__restrict__ 
                  (mw[j] & ((1u << max(low[j], 0)) - 1u)) == 0;
         any = any || fit[j];
         if (tid == 0 && NW * n_blk + j < nn)
-            redo[blockIdx.z * nn * nt + block_of(NW * n_blk + j, t_tile, nn, nt)] = fit[j] ? 0 : 1;
+            redo[blockIdx.z * nn * nt + (NW == 1 ? (int)blockIdx.x
+                                                 : block_of(NW * n_blk + j, t_tile, nn, nt))] =
+                fit[j] ? 0 : 1;
     }
     if (!any) {
         wait_vm<0>();   // no DMA in flight when the block gives its LDS back
@@ -1499,8 +1510,8 @@ int q48_launch_gemm_prepare(q48_ctx *c, void *Wp, const int64_t *W, int N, int K
     uint32_t *m = (uint32_t *)(p + (size_t)nn * steps * 8 * PLANE);
     hipLaunchKernelGGL(k_tile_shift, dim3(nn, tile_parts(K, steps)), dim3(1024), 0, c->stream, m,
                        W, N, K, steps);
-    hipLaunchKernelGGL(k_planes, dim3(nn * steps), dim3(256), 0, c->stream, p, m, W, N, K,
-                       steps, steps, 1);
+    hipLaunchKernelGGL(k_planes<true>, dim3(nn * steps), dim3(256), 0, c->stream, p, m, W, N, K,
+                       steps, 1);
     return (int)hipGetLastError();
 }
 
@@ -1559,15 +1570,15 @@ int q48_launch_gemm_i8(q48_ctx *c, int64_t *Y, const int64_t *W, const int64_t *
     if (planes) {
         uint8_t *Xp = (uint8_t *)(ws + flags + part), *Wp = Xp + xpl;
         uint32_t *Xm = (uint32_t *)(Wp + wpl), *Wm = (uint32_t *)((char *)Xm + xms);
-        hipLaunchKernelGGL(k_planes, dim3(nt * (steps + 1)), dim3(256), 0, c->stream, Xp, Xm,
-                           X, T, K, steps, steps + 1, 0);
+        hipLaunchKernelGGL(k_planes<false>, dim3(nt * (steps + 1)), dim3(256), 0, c->stream, Xp,
+                           Xm, X, T, K, steps, 0);
         if (Wpre) {
             // planes from q48_launch_gemm_prepare: masks after the planes
             Wp = (uint8_t *)Wpre;
             Wm = (uint32_t *)(Wp + (size_t)nn * steps * 8 * PLANE);
         } else {
-            hipLaunchKernelGGL(k_planes, dim3(nn * steps), dim3(256), 0, c->stream, Wp, Wm, W, N,
-                               K, steps, steps, 0);
+            hipLaunchKernelGGL(k_planes<true>, dim3(nn * steps), dim3(256), 0, c->stream, Wp, Wm,
+                               W, N, K, steps, 0);
         }
         // one or two row tiles a block, by rounds of blocks over the compute
         // units: a block of two takes 1.78 to 1.87 times one of one (2048 x 11264
